@@ -46,7 +46,10 @@ template <> struct RT<PT_FLOAT16> {
     __device__ static C cv(S s) { return f16_to_float(s); }
 };
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at any element boundary: gfx950 runs global_load/store_dwordx4 at
+// every byte address, so a row whose pitch is not a multiple of 16 bytes is
+// read with the same instructions as an aligned one.
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4), aligned(2)));
 
 // 16-byte chunk of a row.  Rows are read exactly once, so the loads are
 // nontemporal: on gfx950 that keeps the HBM stream at a higher rate than
@@ -1379,29 +1382,122 @@ __global__ __launch_bounds__(256) void k_column_final(const GenAcc *__restrict__
     gen_finish(a, p, out, i);
 }
 
-// Typed column reductions (floating inputs; sum, mean, prod, max, min) of a
-// contiguous [outer, n, inner] input along n.  A 256-thread block owns
+// What one output keeps while a lane folds its elements in (add), and the
+// state P in which lanes, waves and slices meet (part, merge).
+template <typename C, int OP> struct Fold {
+    using P = C;
+    Acc<C, OP> a;
+    __device__ void begin(C) {}
+    __device__ void add(C v, int) { a.add(v, 0); }
+    __device__ P part(size_t) const { return a.s; }
+    __device__ static P none() { return Acc<C, OP>().s; }
+    __device__ static P merge(P x, P y)
+    {
+        Acc<C, OP> p, q;
+        p.s = x;
+        q.s = y;
+        p.merge(q);
+        return p.s;
+    }
+};
+template <typename C, int OP> struct ArgFold {
+    using P = Acc<C, OP>;
+    Acc<C, OP> a;
+    __device__ void begin(C) {}
+    __device__ void add(C v, int i) { a.add(v, i); }
+    __device__ P part(size_t) const { return a; }
+    __device__ static P none() { return P(); }
+    __device__ static P merge(P x, P y)
+    {
+        x.merge(y);
+        return x;
+    }
+};
+template <typename C> struct Fold<C, R_ARGMAX> : ArgFold<C, R_ARGMAX> {};
+template <typename C> struct Fold<C, R_ARGMIN> : ArgFold<C, R_ARGMIN> {};
+// Moments in double, as sums of the deviations from the lane's first value
+// and of their squares: two additions and a multiplication an element where
+// Welford's step has a division.  The shift is one of the values, so the
+// subtraction at the end loses at most a factor of the lane's count
+// ((shift - mean)^2 <= count x variance), and an infinite or NaN element
+// still makes the result NaN (inf - inf).
+template <typename C> struct Fold<C, R_VAR> {
+    using P = Mom;
+    double shift = 0, s = 0, q = 0;
+    __device__ void begin(C v) { shift = (double)v; }
+    __device__ void add(C v, int)
+    {
+        const double d = (double)v - shift;
+        s = s + d;
+        q = q + d * d;
+    }
+    __device__ P part(size_t n) const
+    {
+        if (n == 0) return none();
+        const double dn = (double)n, m2 = q - s * (s / dn);
+        return Mom{dn, shift + s / dn, m2 < 0.0 ? 0.0 : m2};
+    }
+    __device__ static P none() { return Mom{0, 0, 0}; }
+    __device__ static P merge(P x, P y) { return mom_combine(x, y); }
+};
+
+template <typename C, int OP>
+__device__ __forceinline__ void fold_store(void *out, int out_dt, size_t i, typename Fold<C, OP>::P p, size_t n,
+                                           int correction, int take_sqrt)
+{
+    if constexpr (OP == R_ARGMAX || OP == R_ARGMIN) {
+        ((int32_t *)out)[i] = p.i;
+    } else if constexpr (OP == R_VAR) {
+        const double var = p.m2 / (double)(n - (size_t)correction);
+        store_out(out, out_dt, i, take_sqrt ? sqrt(var) : var);
+    } else if constexpr (OP == R_MEAN) {
+        store_out(out, out_dt, i, p / (C)n);
+    } else {
+        store_out(out, out_dt, i, p);
+    }
+}
+
+// Typed column reductions (floating inputs) of a contiguous
+// [outer, n, inner] input along n.  A 256-thread block owns
 // 64 * V adjacent columns; its four waves take interleaved rows of the
 // block's row slice (adjacent rows in flight together), each lane keeping V
 // columns in registers, and meet in LDS in wave order.  With one slice per
 // column the block writes the result; otherwise it writes a partial per
-// slice and k_col_final_t merges them in slice order.
+// slice and k_col_final_t merges them in slice order.  Rows need no
+// alignment; the lane that straddles the last column loads its columns one
+// by one.
+// Bound by HBM: [20000, 784] fp32 is 62.7 MB.  Argmax and variance took
+// 153 us each on the generic kernels (a 120-byte state of every dtype, one
+// element per lane and load); sum, max, argmax and variance of it one after
+// another went from 359 to 124 us.
 template <int DT, int OP, int V>
 __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ xin, size_t n, size_t inner,
                                                       size_t slice, void *__restrict__ out, int out_dt,
-                                                      typename RT<DT>::C *__restrict__ partial)
+                                                      int correction, int take_sqrt,
+                                                      typename Fold<typename RT<DT>::C, OP>::P *__restrict__ partial)
 {
     using S = typename RT<DT>::S;
     using C = typename RT<DT>::C;
+    using F = Fold<C, OP>;
+    using P = typename F::P;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t col = ((size_t)blockIdx.x * 64 + lane) * V;
     const size_t split = blockIdx.y, o = blockIdx.z;
     const size_t lo = split * slice;
     const size_t hi = lo + slice < n ? lo + slice : n;
-    Acc<C, OP> acc[V];
-    if (col < inner) {
+    const int valid = col >= inner ? 0 : inner - col < (size_t)V ? (int)(inner - col) : V;
+    F acc[V];
+    size_t taken = 0;  // rows this wave has folded in
+    if (valid == V) {
         const S *x = (const S *)xin + o * n * inner + col;
         size_t r = lo + wave;
+        if (r < hi) taken = (hi - r + 3) / 4;
+        if constexpr (OP == R_VAR) {
+            if (r < hi) {
+#pragma unroll
+                for (int k = 0; k < V; k++) acc[k].begin(RT<DT>::cv(x[r * inner + k]));
+            }
+        }
         for (; r + 12 < hi; r += 16) {
             C v[4][V];
 #pragma unroll
@@ -1412,38 +1508,48 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
 #pragma unroll
             for (int u = 0; u < 4; u++)
 #pragma unroll
-                for (int k = 0; k < V; k++) acc[k].add(v[u][k], 0);
+                for (int k = 0; k < V; k++) acc[k].add(v[u][k], (int)(r + 4 * u));
         }
         for (; r < hi; r += 4) {
             C v[V];
             if constexpr (V > 1) load_chunk<DT, V>(x + r * inner, v);
             else v[0] = RT<DT>::cv(x[r * inner]);
 #pragma unroll
-            for (int k = 0; k < V; k++) acc[k].add(v[k], 0);
+            for (int k = 0; k < V; k++) acc[k].add(v[k], (int)r);
         }
+    } else if (valid) {
+        const S *x = (const S *)xin + o * n * inner + col;
+        size_t r = lo + wave;
+        if (r < hi) taken = (hi - r + 3) / 4;
+#pragma unroll
+        for (int k = 0; k < V; k++)
+            if (k < valid && r < hi) acc[k].begin(RT<DT>::cv(x[r * inner + k]));
+        for (; r < hi; r += 4)
+#pragma unroll
+            for (int k = 0; k < V; k++)
+                if (k < valid) acc[k].add(RT<DT>::cv(x[r * inner + k]), (int)r);
     }
-    __shared__ C part[3][64 * V];
+    __shared__ LdsSlot<P> part[3][64 * V];
     if (wave > 0)
 #pragma unroll
-        for (int k = 0; k < V; k++) part[wave - 1][lane * V + k] = acc[k].s;
-    __syncthreads();
-    if (wave != 0 || col >= inner) return;
-#pragma unroll
-    for (int w = 0; w < 3; w++)
-#pragma unroll
         for (int k = 0; k < V; k++) {
-            Acc<C, OP> b;
-            b.s = part[w][lane * V + k];
-            acc[k].merge(b);
+            const P p = acc[k].part(taken);
+            memcpy(part[wave - 1][k * 64 + lane].raw, &p, sizeof(P));
         }
+    __syncthreads();
+    if (wave != 0) return;
 #pragma unroll
     for (int k = 0; k < V; k++) {
-        if (partial) {
-            partial[(o * gridDim.y + split) * inner + col + k] = acc[k].s;
-        } else {
-            C r = OP == R_MEAN ? acc[k].s / (C)n : acc[k].s;
-            store_out(out, out_dt, o * inner + col + k, r);
+        if (k >= valid) continue;
+        P a = acc[k].part(taken);
+#pragma unroll
+        for (int w = 0; w < 3; w++) {
+            P b;
+            memcpy(&b, part[w][k * 64 + lane].raw, sizeof(P));
+            a = F::merge(a, b);
         }
+        if (partial) partial[(o * gridDim.y + split) * inner + col + k] = a;
+        else fold_store<C, OP>(out, out_dt, o * inner + col + k, a, n, correction, take_sqrt);
     }
 }
 
@@ -1451,51 +1557,157 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
 // merges a contiguous quarter of the slices for 64 columns, then wave 0
 // merges the quarters in order.
 template <int DT, int OP>
-__global__ __launch_bounds__(256) void k_col_final_t(const typename RT<DT>::C *__restrict__ partial,
-                                                     size_t splits, size_t inner, size_t n,
-                                                     void *__restrict__ out, int out_dt)
+__global__ __launch_bounds__(256) void k_col_final_t(
+    const typename Fold<typename RT<DT>::C, OP>::P *__restrict__ partial, size_t splits, size_t inner, size_t n,
+    void *__restrict__ out, int out_dt, int correction, int take_sqrt)
 {
     using C = typename RT<DT>::C;
+    using F = Fold<C, OP>;
+    using P = typename F::P;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t col = (size_t)blockIdx.x * 64 + lane, o = blockIdx.y;
     const size_t q = (splits + 3) / 4;
     const size_t lo = wave * q, hi = lo + q < splits ? lo + q : splits;
-    Acc<C, OP> acc;
+    P acc = F::none();
     if (col < inner) {
-        const C *p = partial + o * splits * inner + col;
+        const P *p = partial + o * splits * inner + col;
         size_t k = lo;
         for (; k + 3 < hi; k += 4) {
-            C v[4];
+            P v[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) v[u] = p[(k + u) * inner];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                Acc<C, OP> b;
-                b.s = v[u];
-                acc.merge(b);
-            }
+            for (int u = 0; u < 4; u++) acc = F::merge(acc, v[u]);
         }
-        for (; k < hi; k++) {
-            Acc<C, OP> b;
-            b.s = p[k * inner];
-            acc.merge(b);
-        }
+        for (; k < hi; k++) acc = F::merge(acc, p[k * inner]);
     }
-    __shared__ C part[3][64];
-    if (wave > 0) part[wave - 1][lane] = acc.s;
+    __shared__ LdsSlot<P> part[3][64];
+    if (wave > 0) memcpy(part[wave - 1][lane].raw, &acc, sizeof(P));
     __syncthreads();
     if (wave != 0 || col >= inner) return;
     for (int w = 0; w < 3; w++) {
-        Acc<C, OP> b;
-        b.s = part[w][lane];
-        acc.merge(b);
+        P b;
+        memcpy(&b, part[w][lane].raw, sizeof(P));
+        acc = F::merge(acc, b);
     }
-    C r = OP == R_MEAN ? acc.s / (C)n : acc.s;
-    store_out(out, out_dt, o * inner + col, r);
+    fold_store<C, OP>(out, out_dt, o * inner + col, acc, n, correction, take_sqrt);
 }
 
-// Global reduction of a contiguous input: stage 1 writes one GenAcc per
-// workgroup (each takes a contiguous slice, so index ties resolve to the
+template <typename P>
+__device__ __forceinline__ P part_shfl(const P &p, int m)
+{
+    if constexpr (std::is_same_v<P, Mom>) {
+        return mom_shfl(p, m);
+    } else if constexpr (std::is_floating_point_v<P>) {
+        return __shfl_xor(p, m, PT_WAVE);
+    } else {
+        P o;
+        o.v = __shfl_xor(p.v, m, PT_WAVE);
+        o.i = __shfl_xor(p.i, m, PT_WAVE);
+        return o;
+    }
+}
+
+// The four waves' states of a 256-thread block, merged (thread 0's value counts).
+template <typename F>
+__device__ __forceinline__ typename F::P fold_block(typename F::P p)
+{
+    using P = typename F::P;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) p = F::merge(p, part_shfl(p, m));
+    __shared__ LdsSlot<P> part[4];
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) memcpy(part[wave].raw, &p, sizeof(P));
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < 4; w++) {
+            P b;
+            memcpy(&b, part[w].raw, sizeof(P));
+            p = F::merge(p, b);
+        }
+    return p;
+}
+
+// Typed reduction of all elements of a contiguous floating input: the grid
+// walks the input in 16-byte chunks, adjacent lanes on adjacent chunks and
+// four chunks a lane in flight, each lane folding the V positions of its
+// chunks into V states.  (The generic kernels give every thread a slice of
+// its own, 32 elements away from its neighbour's: a wave-wide load then
+// touches 64 lines.)  A single block writes the result; otherwise
+// k_glob_final_t merges the blocks' states.
+template <int DT, int OP>
+__global__ __launch_bounds__(256) void k_glob_reduce_t(
+    const void *__restrict__ xin, size_t count, typename Fold<typename RT<DT>::C, OP>::P *__restrict__ partial,
+    void *__restrict__ out, int out_dt, int correction, int take_sqrt)
+{
+    using S = typename RT<DT>::S;
+    using C = typename RT<DT>::C;
+    using F = Fold<C, OP>;
+    using P = typename F::P;
+    constexpr int V = RT<DT>::V, U = 4;
+    const S *x = (const S *)xin;
+    const size_t step = (size_t)gridDim.x * 256 * V;
+    size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
+    F acc[V];
+    size_t full = 0;  // whole chunks this lane has folded in
+    int tail = 0;     // elements of the chunk that ends the input
+    if (i < count) {
+        const C first = RT<DT>::cv(x[i]);
+#pragma unroll
+        for (int k = 0; k < V; k++) acc[k].begin(first);
+    }
+    for (; i + (U - 1) * step + V <= count; i += U * step) {
+        C v[U][V];
+#pragma unroll
+        for (int u = 0; u < U; u++) load_chunk<DT, V>(x + i + u * step, v[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 0; k < V; k++) acc[k].add(v[u][k], (int)(i + u * step + k));
+        full += U;
+    }
+    for (; i < count; i += step) {
+        if (i + V <= count) {
+            C v[V];
+            load_chunk<DT, V>(x + i, v);
+#pragma unroll
+            for (int k = 0; k < V; k++) acc[k].add(v[k], (int)(i + k));
+            full++;
+        } else {
+            tail = (int)(count - i);
+#pragma unroll
+            for (int k = 0; k < V; k++)
+                if (k < tail) acc[k].add(RT<DT>::cv(x[i + k]), (int)(i + k));
+        }
+    }
+    P p[V];
+#pragma unroll
+    for (int k = 0; k < V; k++) p[k] = acc[k].part(full + (k < tail ? 1 : 0));
+#pragma unroll
+    for (int h = V / 2; h >= 1; h >>= 1)
+#pragma unroll
+        for (int k = 0; k < h; k++) p[k] = F::merge(p[k], p[k + h]);
+    const P r = fold_block<F>(p[0]);
+    if (threadIdx.x != 0) return;
+    if (partial) partial[blockIdx.x] = r;
+    else fold_store<C, OP>(out, out_dt, 0, r, count, correction, take_sqrt);
+}
+
+template <int DT, int OP>
+__global__ __launch_bounds__(256) void k_glob_final_t(
+    const typename Fold<typename RT<DT>::C, OP>::P *__restrict__ partial, int parts, size_t count,
+    void *__restrict__ out, int out_dt, int correction, int take_sqrt)
+{
+    using C = typename RT<DT>::C;
+    using F = Fold<C, OP>;
+    typename F::P p = F::none();
+    for (int i = threadIdx.x; i < parts; i += 256) p = F::merge(p, partial[i]);
+    p = fold_block<F>(p);
+    if (threadIdx.x == 0) fold_store<C, OP>(out, out_dt, 0, p, count, correction, take_sqrt);
+}
+
+// Global reduction of a contiguous integer or bool input (and all / any of
+// every dtype): stage 1 writes one GenAcc per workgroup (each takes a contiguous slice, so index ties resolve to the
 // lowest index), stage 2 merges them in order.
 __global__ __launch_bounds__(256) void k_global_partial(const void *__restrict__ x, int op, int dt,
                                                         size_t count, size_t base,
@@ -1705,22 +1917,25 @@ static int result_dtype(int dtype, int rop)
     return dtype;
 }
 
-// Column launcher of k_col_reduce_t: whole-16-byte column packs when the
-// row pitch and base keep them aligned; when the column blocks cannot fill
-// the GPU the rows are split into slices (at least 64 rows each, at most
-// 128 slices) merged by k_col_final_t.
+// Column launcher of k_col_reduce_t.  Columns are read in 16-byte packs
+// unless a row holds less than half a block of them (below that the lanes
+// left idle cost more than the narrower loads).  When the column blocks
+// cannot fill the GPU the rows are split into slices (at least 64 rows each,
+// at most 128 slices) merged by k_col_final_t; the number of slices counts
+// unaligned columns one by one, so the scratch they take stays within the
+// no-allocation entry's megabyte for the same calls.
 template <int DT, int OP>
 static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inner, void *out, int out_dt,
-                               hipStream_t s)
+                               int correction, int take_sqrt, hipStream_t s)
 {
-    using C = typename RT<DT>::C;
+    using P = typename Fold<typename RT<DT>::C, OP>::P;
     constexpr int V = RT<DT>::V;
-    const bool vec = inner % V == 0 && aligned16(x);
-    const size_t cols_per_block = vec ? 64 * V : 64;
-    const size_t col_blocks = (inner + cols_per_block - 1) / cols_per_block;
+    const bool packed = inner % V == 0 && aligned16(x);
+    const bool vec = packed || inner >= 32 * V;
+    const size_t split_blocks = (inner + (packed ? 64 * V : 64) - 1) / (packed ? 64 * V : 64);
     size_t splits = 1;
-    if (col_blocks * outer < 1024) {
-        splits = (2048 + col_blocks * outer - 1) / (col_blocks * outer);
+    if (split_blocks * outer < 1024) {
+        splits = (2048 + split_blocks * outer - 1) / (split_blocks * outer);
         size_t max_splits = n / 64;
         if (splits > max_splits) splits = max_splits;
         if (splits > 128) splits = 128;
@@ -1728,15 +1943,18 @@ static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inn
     }
     const size_t slice = (n + splits - 1) / splits;
     splits = (n + slice - 1) / slice;
-    C *partial = nullptr;
-    if (splits > 1) PT_TRY(scratch_alloc((void **)&partial, sizeof(C) * outer * splits * inner, s));
-    dim3 grid((unsigned)col_blocks, (unsigned)splits, (unsigned)outer);
-    if (vec) k_col_reduce_t<DT, OP, V><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, partial);
-    else k_col_reduce_t<DT, OP, 1><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, partial);
+    P *partial = nullptr;
+    if (splits > 1) PT_TRY(scratch_alloc((void **)&partial, sizeof(P) * outer * splits * inner, s));
+    const size_t cols_per_block = vec ? 64 * V : 64;
+    dim3 grid((unsigned)((inner + cols_per_block - 1) / cols_per_block), (unsigned)splits, (unsigned)outer);
+    if (vec)
+        k_col_reduce_t<DT, OP, V><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, correction, take_sqrt, partial);
+    else
+        k_col_reduce_t<DT, OP, 1><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, correction, take_sqrt, partial);
     hipError_t e1 = hipGetLastError(), e2 = hipSuccess;
     if (splits > 1) {
         k_col_final_t<DT, OP><<<dim3((unsigned)((inner + 63) / 64), (unsigned)outer), 256, 0, s>>>(
-            partial, splits, inner, n, out, out_dt);
+            partial, splits, inner, n, out, out_dt, correction, take_sqrt);
         e2 = hipGetLastError();
         scratch_free(partial, s);
     }
@@ -1745,29 +1963,53 @@ static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inn
     return PT_OK;
 }
 
-template <int DT>
-static int launch_cols_dt(int rop, const void *x, size_t outer, size_t n, size_t inner, void *out, int out_dt,
-                          hipStream_t s)
+// Launcher of k_glob_reduce_t: a block per 4 chunks of each of its lanes, up
+// to four blocks a CU.
+template <int DT, int OP>
+static pt_status launch_glob_t(const void *x, size_t count, void *out, int out_dt, int correction, int take_sqrt,
+                               hipStream_t s)
 {
-    switch (rop) {
-    case R_SUM: return launch_cols_t<DT, R_SUM>(x, outer, n, inner, out, out_dt, s);
-    case R_MEAN: return launch_cols_t<DT, R_MEAN>(x, outer, n, inner, out, out_dt, s);
-    case R_PROD: return launch_cols_t<DT, R_PROD>(x, outer, n, inner, out, out_dt, s);
-    case R_MAX: return launch_cols_t<DT, R_MAX>(x, outer, n, inner, out, out_dt, s);
-    case R_MIN: return launch_cols_t<DT, R_MIN>(x, outer, n, inner, out, out_dt, s);
+    using P = typename Fold<typename RT<DT>::C, OP>::P;
+    constexpr size_t per_block = 256 * 4 * RT<DT>::V;
+    size_t blocks = (count + per_block - 1) / per_block;
+    if (blocks > 1024) blocks = 1024;
+    P *partial = nullptr;
+    if (blocks > 1) PT_TRY(scratch_alloc((void **)&partial, sizeof(P) * blocks, s));
+    k_glob_reduce_t<DT, OP><<<(unsigned)blocks, 256, 0, s>>>(x, count, partial, out, out_dt, correction, take_sqrt);
+    hipError_t e1 = hipGetLastError(), e2 = hipSuccess;
+    if (blocks > 1) {
+        k_glob_final_t<DT, OP><<<1, 256, 0, s>>>(partial, (int)blocks, count, out, out_dt, correction, take_sqrt);
+        e2 = hipGetLastError();
+        scratch_free(partial, s);
     }
-    return -1;
+    PT_TRY(check_hip(e1, "global reduction (partials)"));
+    PT_TRY(check_hip(e2, "global reduction (final)"));
+    return PT_OK;
 }
 
-// Returns -1 when the typed column path does not cover (dtype, op).
-static int launch_cols(int dt, int rop, const void *x, size_t outer, size_t n, size_t inner, void *out,
-                       int out_dt, hipStream_t s)
+// f(integral constants of dtype and op) for the floating dtypes and every
+// typed op; -1 when the typed kernels do not cover (dtype, op).
+template <typename F>
+static int typed_reduction(int dt, int rop, F f)
 {
+    auto with_op = [&](auto D) -> int {
+        switch (rop) {
+        case R_SUM: return f(D, std::integral_constant<int, R_SUM>{});
+        case R_MEAN: return f(D, std::integral_constant<int, R_MEAN>{});
+        case R_PROD: return f(D, std::integral_constant<int, R_PROD>{});
+        case R_MAX: return f(D, std::integral_constant<int, R_MAX>{});
+        case R_MIN: return f(D, std::integral_constant<int, R_MIN>{});
+        case R_ARGMAX: return f(D, std::integral_constant<int, R_ARGMAX>{});
+        case R_ARGMIN: return f(D, std::integral_constant<int, R_ARGMIN>{});
+        case R_VAR: return f(D, std::integral_constant<int, R_VAR>{});
+        }
+        return -1;
+    };
     switch (dt) {
-    case PT_FLOAT32: return launch_cols_dt<PT_FLOAT32>(rop, x, outer, n, inner, out, out_dt, s);
-    case PT_FLOAT64: return launch_cols_dt<PT_FLOAT64>(rop, x, outer, n, inner, out, out_dt, s);
-    case PT_BFLOAT16: return launch_cols_dt<PT_BFLOAT16>(rop, x, outer, n, inner, out, out_dt, s);
-    case PT_FLOAT16: return launch_cols_dt<PT_FLOAT16>(rop, x, outer, n, inner, out, out_dt, s);
+    case PT_FLOAT32: return with_op(std::integral_constant<int, PT_FLOAT32>{});
+    case PT_FLOAT64: return with_op(std::integral_constant<int, PT_FLOAT64>{});
+    case PT_BFLOAT16: return with_op(std::integral_constant<int, PT_BFLOAT16>{});
+    case PT_FLOAT16: return with_op(std::integral_constant<int, PT_FLOAT16>{});
     }
     return -1;
 }
@@ -1836,6 +2078,15 @@ static pt_status reduce_driver(const void *input, void *output, int dtype, int r
     }
     bool contiguous = is_row_major(shape, strides, ndims);
     if (axis < 0 && contiguous) {
+        int st = typed_reduction(dtype, rop, [&](auto D, auto O) -> int {
+            return launch_glob_t<decltype(D)::value, decltype(O)::value>(xb, total, output, out_dt, correction,
+                                                                         take_sqrt, s);
+        });
+        if (st >= 0) {
+            PT_TRY((pt_status)st);
+            counters().global_reduce_calls++;
+            return PT_OK;
+        }
         int parts = (int)((total + 8191) / 8192);
         if (parts > 1024) parts = 1024;
         if (parts < 1) parts = 1;
@@ -1856,7 +2107,10 @@ static pt_status reduce_driver(const void *input, void *output, int dtype, int r
         for (int d = 0; d < axis; d++) outer *= (size_t)shape[d];
         for (int d = axis + 1; d < ndims; d++) inner *= (size_t)shape[d];
         if (outer <= 65535 && count <= (size_t)INT32_MAX) {
-            int st = launch_cols(dtype, rop, xb, outer, count, inner, output, out_dt, s);
+            int st = typed_reduction(dtype, rop, [&](auto D, auto O) -> int {
+                return launch_cols_t<decltype(D)::value, decltype(O)::value>(xb, outer, count, inner, output, out_dt,
+                                                                             correction, take_sqrt, s);
+            });
             if (st >= 0) {
                 PT_TRY((pt_status)st);
                 counters().column_reduce_calls++;

@@ -1,0 +1,112 @@
+"""GPU parity of the typed reductions over non-last axes and over all
+elements: argmax / argmin / variance along columns and every op over a whole
+tensor, at the edges of their blocks (columns per block, a straddling last
+lane, one and several row slices, whole and partial chunks, one and several
+blocks), against the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+DTS = [O.F32, O.F64, O.BF16, O.F16]
+NAMES = {O.F32: "f32", O.F64: "f64", O.BF16: "bf16", O.F16: "f16"}
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gpu_util
+    from phptensors import _abi
+    _abi.load()
+    _abi.check(_abi.load().pt_init(), "init")
+    return gpu_util
+
+
+def _ints(shape, dt, seed):
+    """Small whole numbers (every sum exact, many ties) with a NaN and both infinities in some columns."""
+    from phptensors import synthetic
+    x = np.round(synthetic.uniform(shape, -40.0, 40.0, seed=seed)).astype(np.float32)
+    return x, O.to_storage(x.astype(np.float64) if dt == O.F64 else x, dt)
+
+
+def _check_var(G, xs, dt, axis):
+    """The deviations are summed in double (relative error below n 2^-53 of the
+    result, n at most 3e5), the result is rounded to the output type once."""
+    x = O.from_storage(xs, dt).astype(np.float64)
+    rtol = 1e-10 if dt == O.F64 else 2.0 ** -23
+    for corr, std in ((0, False), (1, True)):
+        if (x.shape[axis] if axis is not None else x.size) <= corr:
+            continue
+        got = np.asarray(G.moments(xs, dt, axis, corr, std), np.float64).ravel()
+        ref = np.atleast_1d(x.std(axis, ddof=corr) if std else x.var(axis, ddof=corr)).ravel()
+        assert np.allclose(got, ref, rtol=rtol, atol=0, equal_nan=True), (corr, std)
+
+
+@pytest.mark.parametrize("dt", DTS, ids=NAMES.get)
+@pytest.mark.parametrize("shape,axis", [((2, 3), 0), ((3, 5, 1), 1), ((130, 31), 0), ((257, 129), 0), ((64, 257), 0),
+                                        ((4097, 1001), 0), ((5, 70, 513), 1), ((20000, 40), 0), ((70, 33000), 0)],
+                         ids=str)
+def test_column_arg_and_variance(G, dt, shape, axis):
+    x, xs = _ints(shape, dt, 11 + shape[0])
+    for op in ("argmax", "argmin"):
+        assert np.array_equal(G.arg_reduce(xs, dt, op, axis), O.arg_reduce(xs, dt, op, axis)), op
+    _check_var(G, xs, dt, axis)
+    for op in ("sum", "max"):
+        got, _ = G.reduce(xs, dt, op, axis)
+        assert np.array_equal(got, O.reduce(xs, dt, op, axis)[0]), op
+
+
+@pytest.mark.parametrize("dt", DTS, ids=NAMES.get)
+@pytest.mark.parametrize("n", [1, 7, 255, 1024, 4096, 4097, 16385, 300001])
+def test_global_reductions(G, dt, n):
+    x, xs = _ints((n,), dt, n)
+    for op in ("argmax", "argmin"):
+        assert np.array_equal(G.arg_reduce(xs, dt, op, None), O.arg_reduce(xs, dt, op, None)), op
+    for op in ("sum", "max", "min"):
+        got, rdt = G.reduce(xs, dt, op, None)
+        ref, rrdt = O.reduce(xs, dt, op, None)
+        assert rdt == rrdt and np.array_equal(got.ravel(), ref.ravel()), op
+    got, _ = G.reduce(xs, dt, "mean", None)
+    assert np.allclose(got.ravel(), O.reduce(xs, dt, "mean", None)[0].ravel(), rtol=2e-7, atol=0)
+    _check_var(G, xs, dt, None)
+
+
+@pytest.mark.parametrize("dt", DTS, ids=NAMES.get)
+@pytest.mark.parametrize("axis", [0, None])
+def test_nonfinite_values(G, dt, axis):
+    """NaN is never taken by arg reductions, a column without any value above
+    -inf (below inf) gives index 0, and NaN or an infinity anywhere makes a
+    variance NaN."""
+    x, _ = _ints((700, 140), dt, 5)
+    x[3, 0] = x[0, 1] = np.nan
+    x[:, 2], x[:, 3], x[:, 4] = -np.inf, np.inf, np.nan
+    x[699, 5], x[0, 6] = np.inf, -np.inf
+    x[:, 7], x[350, 7] = -np.inf, np.nan
+    xs = O.to_storage(x.astype(np.float64) if dt == O.F64 else x, dt)
+    for op in ("argmax", "argmin"):
+        assert np.array_equal(G.arg_reduce(xs, dt, op, axis), O.arg_reduce(xs, dt, op, axis)), op
+    got = np.asarray(G.moments(xs, dt, axis)).ravel()
+    if axis is None:
+        assert np.isnan(got[0])
+    else:
+        assert np.all(np.isnan(got[:8])) and np.all(np.isfinite(got[8:]))
+
+
+def test_variance_far_from_zero(G):
+    """A mean far above the spread, and a first value far from the others."""
+    from phptensors import synthetic
+    x = synthetic.normal((5000, 70), 1e4, 1.0, seed=9).astype(np.float32)
+    x[0, 10:20] = -3e4
+    for axis in (0, None):
+        _check_var(G, x, O.F32, axis)
+
+
+def test_global_reduction_of_an_offset_view(G):
+    """A base that is no multiple of 16 bytes."""
+    x, xs = _ints((9001,), O.BF16, 3)
+    for off in (1, 3, 8):
+        from phptensors import CudaArray
+        v = CudaArray.fromNumpy(xs, "bfloat16").slice([off, None])
+        assert v.sum().item() == float(x[off:].sum())
+        assert v.argMax().item() == int(np.argmax(x[off:]))
