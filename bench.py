@@ -256,12 +256,12 @@ def eager_family(steps, warmup):
     ops = {
         "mul_row_broadcast": (lambda st: lib.pt_broadcast(y.ptr, A.FLOAT32, row_b, 0, z.ptr, A.FLOAT32, dense, 0,
                                                           m.ptr, A.FLOAT32, A.OP["mul"], shape, 2, st),
-                              2 * big + n * 4, "k_binary_f32_rows"),
+                              2 * big + n * 4, "k_binary_vec<f32>"),
         "add": (lambda st: lib.pt_broadcast(x.ptr, A.FLOAT32, dense, 0, m.ptr, A.FLOAT32, dense, 0,
                                             s_.ptr, A.FLOAT32, A.OP["add"], shape, 2, st),
-                3 * big, "k_binary_f32_contig"),
+                3 * big, "k_binary_vec<f32>"),
         "tanh": (lambda st: lib.pt_unary(s_.ptr, A.FLOAT32, dense, 0, t.ptr, A.OP["tanh"], shape, 2, st),
-                 2 * big, "k_unary_f32_contig"),
+                 2 * big, "k_unary_vec<f32>"),
     }
     results = {}
     for name, (fn, nbytes, kernel) in ops.items():

@@ -3,10 +3,10 @@
 //
 // The host collapses the output shape first (adjacent dimensions merge
 // when every operand's strides allow it; size-1 dimensions drop), so most
-// broadcasts reach the kernels as 1-2 dimensions.  All-contiguous operands
-// of one dtype take a vectorized path (16-byte loads and stores); every
-// other layout and dtype mix runs the generic path, which decodes the
-// collapsed index and converts through the compute type.
+// broadcasts reach the kernels as 1-2 dimensions.  Floating operands of one
+// 32- or 16-bit dtype in such layouts take the vector path (16-byte loads and
+// stores); every other layout and dtype mix runs the generic path, which
+// decodes the collapsed index and converts through the compute type.
 //
 // Op semantics follow the reference functors (cuda_op_functors.cuh:12-449):
 // operands are converted to the output dtype (float for f16/bf16 outputs),
@@ -20,14 +20,10 @@
 #include <math.h>
 #include <string.h>
 
+#include <initializer_list>
+#include <utility>
+
 namespace pt {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Streaming 16-byte accesses: operands read once and results written once
-// bypass cache retention (nontemporal), which keeps HBM streams at full rate.
-__device__ __forceinline__ f32x4 ld_stream(const float *p) { return __builtin_nontemporal_load((const f32x4 *)p); }
-__device__ __forceinline__ void st_stream(float *p, f32x4 v) { __builtin_nontemporal_store(v, (f32x4 *)p); }
 
 struct EwShape {
     int ndims;
@@ -256,70 +252,246 @@ __global__ __launch_bounds__(256) void k_binary(const void *__restrict__ a, int 
     }
 }
 
-// All-contiguous float32 fast path: 4 elements per thread per step.
-__global__ __launch_bounds__(256) void k_binary_f32_contig(const float *__restrict__ a,
-                                                           const float *__restrict__ b,
-                                                           float *__restrict__ out, int op,
-                                                           long long n, int b_scalar, float scalar,
-                                                           int reverse)
+// ---------------------------------------------------- 16-byte vector path
+// Floating outputs of 32 and 16 bits: each thread makes 16 bytes of the
+// (contiguous) output, 4 or 8 elements, from operands that are contiguous
+// too, walk the rows of a collapsed [rows, cols] output (column stride 1, any
+// row stride, 0 for a broadcast row), hold one value per row (column stride
+// 0), or are one immediate.  The output is cut into chunks as one flat
+// array, so that chunks of it and of contiguous operands stay aligned
+// whatever cols is; a chunk that crosses a row's end takes the other kinds of
+// operand element by element.  All of these kernels are bound by HBM: one
+// element per thread with an index decode, a dtype switch and a 2-byte load
+// took 91 us for x + b on [8000, 3001] bf16 (96 MB); the six calls of an
+// eager activation on it went from 499 to 150 us.
+enum { OPND_FLAT = 0, OPND_IMM, OPND_ROWS, OPND_COL, OPND_ANY = -1 };
+struct Opnd {
+    const void *p;
+    int mode;
+    unsigned rs;  // row stride (OPND_ROWS, OPND_COL)
+    float imm;
+};
+
+// A thread's chunk: elements i .. i + V - 1 of the output, element i being
+// (r, c) of [rows, cols] where an operand needs that; `valid` of them exist.
+// `whole`: every chunk of the block is complete, `even`: and none crosses a
+// row's end, each one scalar test a block.
+template <int V>
+struct ChunkPos {
+    size_t i;
+    int valid;
+    bool whole, even;
+    unsigned r = 0, c = 0;
+    __device__ __forceinline__ ChunkPos(size_t total, unsigned cols, bool rowwise)
+    {
+        const size_t b = (size_t)blockIdx.x * (256 * V);
+        i = b + threadIdx.x * V;
+        whole = b + 256 * V <= total;
+        valid = whole || i + V <= total ? V : i < total ? (int)(total - i) : 0;
+        even = whole && cols % V == 0;
+        if (rowwise) {  // (the host keeps such outputs below 2^31 elements)
+            r = (unsigned)i / cols;
+            c = (unsigned)i - r * cols;
+        }
+    }
+};
+
+// N bytes at any element boundary (16 at a time where N allows).
+typedef unsigned int u32x4v __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned int u32x2v __attribute__((ext_vector_type(2), aligned(1)));
+template <int N, bool NT>
+__device__ __forceinline__ void ld_bytes(void *dst, const void *src)
 {
-    long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    const long long stride = (long long)gridDim.x * blockDim.x * 4;
-    for (; i < n; i += stride) {
-        if (i + 4 <= n) {
-            f32x4 x = ld_stream(a + i);
-            f32x4 y = b_scalar ? (f32x4){scalar, scalar, scalar, scalar} : ld_stream(b + i);
-            f32x4 r;
-            if (reverse) {
-                r.x = bin_op<float>(op, y.x, x.x); r.y = bin_op<float>(op, y.y, x.y);
-                r.z = bin_op<float>(op, y.z, x.z); r.w = bin_op<float>(op, y.w, x.w);
-            } else {
-                r.x = bin_op<float>(op, x.x, y.x); r.y = bin_op<float>(op, x.y, y.y);
-                r.z = bin_op<float>(op, x.z, y.z); r.w = bin_op<float>(op, x.w, y.w);
-            }
-            st_stream(out + i, r);
+    if constexpr (N >= 16) {
+#pragma unroll
+        for (int q = 0; q < N / 16; q++) {
+            u32x4v t;
+            if constexpr (NT) t = __builtin_nontemporal_load((const u32x4v *)src + q);
+            else t = ((const u32x4v *)src)[q];
+            memcpy((char *)dst + 16 * q, &t, 16);
+        }
+    } else if constexpr (N == 8) {
+        const u32x2v t = *(const u32x2v *)src;
+        memcpy(dst, &t, 8);
+    } else {
+        memcpy(dst, src, N);
+    }
+}
+
+// Elements of an operand for the chunk at q, as they lie in memory (T: an
+// unsigned type of the element's size).  MODE: the operand's layout where
+// the kernel is built for it (no branch around its load), else OPND_ANY.
+template <int MODE, typename T, int V, bool NT>
+__device__ __forceinline__ void fetch(const Opnd &o, const ChunkPos<V> &q, unsigned cols, T (&v)[V])
+{
+    const T *p = (const T *)o.p;
+    const int mode = MODE == OPND_ANY ? o.mode : MODE;
+    unsigned r = q.r, c = q.c;
+    if (mode == OPND_IMM) return;
+    if (mode == OPND_FLAT) {
+        if (q.whole) {
+            ld_bytes<V * sizeof(T), NT>(v, p + q.i);
         } else {
-            for (long long j = i; j < n; j++) {
-                float x = a[j], y = b_scalar ? scalar : b[j];
-                out[j] = reverse ? bin_op<float>(op, y, x) : bin_op<float>(op, x, y);
+#pragma unroll
+            for (int k = 0; k < V; k++) v[k] = k < q.valid ? p[q.i + k] : (T)0;
+        }
+    } else if (q.even || (c + V <= cols && q.valid == V)) {
+        if (mode == OPND_ROWS) {
+            ld_bytes<V * sizeof(T), false>(v, p + (size_t)r * o.rs + c);
+        } else {
+            const T t = p[(size_t)r * o.rs];
+#pragma unroll
+            for (int k = 0; k < V; k++) v[k] = t;
+        }
+    } else {
+        const unsigned cs = mode == OPND_ROWS ? 1u : 0u;
+#pragma unroll
+        for (int k = 0; k < V; k++) {
+            v[k] = k < q.valid ? p[(size_t)r * o.rs + c * cs] : (T)0;
+            if (++c == cols) {
+                c = 0;
+                r++;
             }
         }
     }
 }
 
-// float32 operands over a 2-D [rows, cols] output (cols a multiple of 4):
-// each operand either walks the row (column stride 1, 16-byte loads) or
-// holds one value per row (column stride 0); its row stride may be 0 (a
-// broadcast row).  Operands read once per output element stream past the
-// caches (nontemporal); broadcast ones use ordinary loads.
-__device__ __forceinline__ f32x4 ld_row4(const float *p, unsigned ro, unsigned c, int inner, bool stream)
+template <int DT> struct VecT;
+template <> struct VecT<PT_FLOAT32> {
+    using T = uint32_t;
+    __device__ static float to(T t) { return __uint_as_float(t); }
+    __device__ static T from(float f) { return __float_as_uint(f); }
+};
+template <> struct VecT<PT_BFLOAT16> {
+    using T = uint16_t;
+    __device__ static float to(T t) { return bf16_to_float(t); }
+    __device__ static T from(float f) { return float_to_bf16(f); }
+};
+template <> struct VecT<PT_FLOAT16> {
+    using T = uint16_t;
+    __device__ static float to(T t) { return f16_to_float(t); }
+    __device__ static T from(float f) { return float_to_f16(f); }
+};
+
+template <int DT, int MODE, int V>
+__device__ __forceinline__ void to_float(const Opnd &o, const typename VecT<DT>::T (&t)[V], float (&v)[V])
 {
-    if (!inner) {
-        const float v = p[ro];
-        return (f32x4){v, v, v, v};
-    }
-    return stream ? ld_stream(p + ro + c) : *(const f32x4 *)(p + ro + c);
+    const bool imm = MODE == OPND_ANY ? o.mode == OPND_IMM : MODE == OPND_IMM;
+#pragma unroll
+    for (int k = 0; k < V; k++) v[k] = imm ? o.imm : VecT<DT>::to(t[k]);
 }
 
-__global__ __launch_bounds__(256) void k_binary_f32_rows(const float *__restrict__ a, const float *__restrict__ b,
-                                                         float *__restrict__ out, int op, unsigned rows,
-                                                         unsigned cols4, unsigned ra, int ia, unsigned rb, int ib,
-                                                         int reverse)
+template <typename T, int V, bool NT>
+__device__ __forceinline__ void put(T *out, const ChunkPos<V> &q, const T (&v)[V])
 {
-    const unsigned g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= rows * cols4) return;
-    const unsigned r = g / cols4, c = (g - r * cols4) * 4;
-    const f32x4 x = ld_row4(a, r * ra, c, ia, ia && ra != 0);
-    const f32x4 y = ld_row4(b, r * rb, c, ib, ib && rb != 0);
-    f32x4 v;
-    if (reverse) {
-        v.x = bin_op<float>(op, y.x, x.x); v.y = bin_op<float>(op, y.y, x.y);
-        v.z = bin_op<float>(op, y.z, x.z); v.w = bin_op<float>(op, y.w, x.w);
+    if (q.whole) {
+        constexpr int N = V * sizeof(T) / 16;
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            u32x4v t;
+            memcpy(&t, (const char *)v + 16 * j, 16);
+            if constexpr (NT) __builtin_nontemporal_store(t, (u32x4v *)(out + q.i) + j);
+            else ((u32x4v *)(out + q.i))[j] = t;
+        }
     } else {
-        v.x = bin_op<float>(op, x.x, y.x); v.y = bin_op<float>(op, x.y, y.y);
-        v.z = bin_op<float>(op, x.z, y.z); v.w = bin_op<float>(op, x.w, y.w);
+#pragma unroll
+        for (int k = 0; k < V; k++)
+            if (k < q.valid) out[q.i + k] = v[k];
     }
-    st_stream(out + (size_t)g * 4, v);
+}
+
+// f(op as an integral constant): the op's dispatch is one scalar branch a
+// thread instead of one an element.
+template <typename F>
+__device__ __forceinline__ void with_bin_op(int op, F f)
+{
+    switch (op) {
+    case PT_OP_ADD: f(std::integral_constant<int, PT_OP_ADD>{}); break;
+    case PT_OP_SUB: f(std::integral_constant<int, PT_OP_SUB>{}); break;
+    case PT_OP_MUL: f(std::integral_constant<int, PT_OP_MUL>{}); break;
+    case PT_OP_DIV: f(std::integral_constant<int, PT_OP_DIV>{}); break;
+    case PT_OP_POW: f(std::integral_constant<int, PT_OP_POW>{}); break;
+    case PT_OP_MAXIMUM: f(std::integral_constant<int, PT_OP_MAXIMUM>{}); break;
+    case PT_OP_MINIMUM: f(std::integral_constant<int, PT_OP_MINIMUM>{}); break;
+    case PT_OP_GT: f(std::integral_constant<int, PT_OP_GT>{}); break;
+    case PT_OP_LT: f(std::integral_constant<int, PT_OP_LT>{}); break;
+    case PT_OP_EQ: f(std::integral_constant<int, PT_OP_EQ>{}); break;
+    case PT_OP_NE: f(std::integral_constant<int, PT_OP_NE>{}); break;
+    case PT_OP_GE: f(std::integral_constant<int, PT_OP_GE>{}); break;
+    case PT_OP_LE: f(std::integral_constant<int, PT_OP_LE>{}); break;
+    }
+}
+
+// DT: the operands' type, DTO: the output's (float32 where 16-bit operands
+// divide).
+template <int DT, int DTO, bool NT, int MA, int MB>
+__global__ __launch_bounds__(256) void k_binary_vec(Opnd a, Opnd b, void *__restrict__ out, int op, size_t total,
+                                                    unsigned cols)
+{
+    using T = typename VecT<DT>::T;
+    using TO = typename VecT<DTO>::T;
+    constexpr int V = 16 / sizeof(T);
+    const ChunkPos<V> q(total, cols, (MA == OPND_ANY ? a.mode : MA) >= OPND_ROWS ||
+                                         (MB == OPND_ANY ? b.mode : MB) >= OPND_ROWS);
+    if (!q.valid) return;
+    T u[V], w[V];
+    fetch<MA, T, V, NT>(a, q, cols, u);
+    fetch<MB, T, V, NT>(b, q, cols, w);
+    float x[V], y[V];
+    TO z[V];
+    to_float<DT, MA>(a, u, x);
+    to_float<DT, MB>(b, w, y);
+    with_bin_op(op, [&](auto O) {
+#pragma unroll
+        for (int k = 0; k < V; k++) z[k] = VecT<DTO>::from(bin_op<float>(decltype(O)::value, x[k], y[k]));
+    });
+    put<TO, V, NT>((TO *)out, q, z);
+}
+
+// where(c, x, y): elements of ESZ bytes moved as bits, a condition of CSZ
+// bytes an element that holds where the bits under `mask` (a float's without
+// its sign) are not all zero.
+template <int N> struct BitsT;
+template <> struct BitsT<1> { using T = uint8_t; };
+template <> struct BitsT<2> { using T = uint16_t; };
+template <> struct BitsT<4> { using T = uint32_t; };
+template <> struct BitsT<8> { using T = uint64_t; };
+
+template <int ESZ, int CSZ, bool NT>
+__global__ __launch_bounds__(256) void k_where_vec(Opnd cond, Opnd x, Opnd y, void *__restrict__ out, uint32_t mask,
+                                                   size_t total, unsigned cols)
+{
+    using T = typename BitsT<ESZ>::T;
+    using CT = typename BitsT<CSZ>::T;
+    constexpr int V = 16 / ESZ;
+    const ChunkPos<V> q(total, cols, cond.mode >= OPND_ROWS || x.mode >= OPND_ROWS || y.mode >= OPND_ROWS);
+    if (!q.valid) return;
+    CT c[V];
+    T u[V], w[V];
+    fetch<OPND_ANY, CT, V, NT>(cond, q, cols, c);
+    fetch<OPND_ANY, T, V, NT>(x, q, cols, u);
+    fetch<OPND_ANY, T, V, NT>(y, q, cols, w);
+#pragma unroll
+    for (int k = 0; k < V; k++) u[k] = ((uint32_t)c[k] & mask) ? u[k] : w[k];
+    put<T, V, NT>((T *)out, q, u);
+}
+
+// Casts between the 32- and 16-bit floating types; V elements are 16 bytes
+// of the wider type.
+template <int DTI, int DTO, bool NT>
+__global__ __launch_bounds__(256) void k_cast_vec(Opnd x, void *__restrict__ out, size_t total, unsigned cols)
+{
+    using TI = typename VecT<DTI>::T;
+    using TO = typename VecT<DTO>::T;
+    constexpr int V = 8;
+    const ChunkPos<V> q(total, cols, x.mode >= OPND_ROWS);
+    if (!q.valid) return;
+    TI t[V];
+    TO z[V];
+    fetch<OPND_ANY, TI, V, NT>(x, q, cols, t);
+#pragma unroll
+    for (int k = 0; k < V; k++) z[k] = VecT<DTO>::from(VecT<DTI>::to(t[k]));
+    put<TO, V, NT>((TO *)out, q, z);
 }
 
 // ------------------------------------------------------------------ unary
@@ -381,24 +553,21 @@ __global__ __launch_bounds__(256) void k_unary(const void *__restrict__ x, int d
 
 // OPC >= 0: the op fixed at compile time (the per-element dispatch folds
 // away); OPC < 0: the op comes from `op`.
-template <int OPC>
-__global__ __launch_bounds__(256) void k_unary_f32_contig(const float *__restrict__ x,
-                                                          float *__restrict__ out, int op_arg, long long n)
+template <int DT, int OPC, bool NT, int MX>
+__global__ __launch_bounds__(256) void k_unary_vec(Opnd x, void *__restrict__ out, int op_arg, size_t total,
+                                                   unsigned cols)
 {
+    using T = typename VecT<DT>::T;
+    constexpr int V = 16 / sizeof(T);
     const int op = OPC >= 0 ? OPC : op_arg;
-    long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    const long long stride = (long long)gridDim.x * blockDim.x * 4;
-    for (; i < n; i += stride) {
-        if (i + 4 <= n) {
-            f32x4 v = ld_stream(x + i);
-            f32x4 r;
-            r.x = unary_f<float>(op, v.x); r.y = unary_f<float>(op, v.y);
-            r.z = unary_f<float>(op, v.z); r.w = unary_f<float>(op, v.w);
-            st_stream(out + i, r);
-        } else {
-            for (long long j = i; j < n; j++) out[j] = unary_f<float>(op, x[j]);
-        }
-    }
+    const ChunkPos<V> q(total, cols, (MX == OPND_ANY ? x.mode : MX) >= OPND_ROWS);
+    if (!q.valid) return;
+    T t[V];
+    fetch<MX, T, V, NT>(x, q, cols, t);
+    T z[V];
+#pragma unroll
+    for (int k = 0; k < V; k++) z[k] = VecT<DT>::from(unary_f<float>(op, VecT<DT>::to(t[k])));
+    put<T, V, NT>((T *)out, q, z);
 }
 
 // --------------------------------------------------------- cast / where
@@ -523,23 +692,54 @@ static long long scalar_as_i64(const pt_scalar_t *s)
     return s->v.i64;
 }
 
-// The 2-D float32 row kernel applies: 1 or 2 collapsed dims, a column
-// count that is a multiple of 4, each operand's column stride 0 or 1, and
-// 16-byte aligned rows for the operands that walk them.
-static bool rows_f32(const EwShape &s, const void *pa, const void *pb, const void *out)
+// An operand of the vector kernels from its collapsed strides st; false when
+// its layout is none of theirs (the generic kernels decode any layout).
+static bool as_opnd(const EwShape &s, const long long *st, const void *p, Opnd &o)
 {
-    if (s.ndims < 1 || s.ndims > 2 || s.total > 0x7fffffffLL) return false;
-    const long long cols = s.shape[s.ndims - 1];
-    if (cols % 4 || ((uintptr_t)out & 15)) return false;
-    const long long ia = s.sa[s.ndims - 1], ib = s.sb[s.ndims - 1];
-    const long long ra = s.ndims == 2 ? s.sa[0] : 0, rb = s.ndims == 2 ? s.sb[0] : 0;
-    if ((ia != 0 && ia != 1) || (ib != 0 && ib != 1)) return false;
-    if (ia == 1 && (((uintptr_t)pa & 15) || ra % 4)) return false;
-    if (ib == 1 && (((uintptr_t)pb & 15) || rb % 4)) return false;
+    o = Opnd{p, OPND_FLAT, 0u, 0.0f};
+    if (s.ndims == 0) return true;
+    if (s.ndims > 2) return false;
+    const long long cols = s.shape[s.ndims - 1], cs = st[s.ndims - 1], rs = s.ndims == 2 ? st[0] : 0;
+    if (cs == 1 && (s.ndims == 1 || rs == cols)) return true;
     const long long rows = s.ndims == 2 ? s.shape[0] : 1;
-    // largest offsets stay in 32 bits
-    if ((rows - 1) * ra + cols > 0x7fffffffLL || (rows - 1) * rb + cols > 0x7fffffffLL) return false;
+    if ((cs != 0 && cs != 1) || s.total > 0x7fffffffLL || rs < 0 || rs > 0x7fffffffLL ||
+        (rows - 1) * rs + cols > 0x7fffffffLL)
+        return false;
+    o.mode = cs == 1 ? OPND_ROWS : OPND_COL;
+    o.rs = (unsigned)rs;
     return true;
+}
+
+static unsigned opnd_cols(const EwShape &s)
+{
+    const long long c = s.ndims ? s.shape[s.ndims - 1] : 1;
+    return c > 0x7fffffffLL ? 1u : (unsigned)c;  // only read where an operand is rowwise (at most 2^31 elements)
+}
+
+// Streaming accesses bypass cache retention (nontemporal) in calls that move
+// a gigabyte or more through aligned chunks: the 256 MB Infinity Cache then
+// holds nothing that the next call could read.  A chain of eager calls (add,
+// gt, where, multiply, add, astype; cached against nontemporal):
+// [8000, 3001] bf16 150 against 166 us, [8000, 3000] fp32 201 against 215,
+// [16000, 8000] bf16 (0.77 GB a call) 690 against 735, [16000, 8001] fp32
+// (1.5 GB a call) 1050 against 992, and tanh of [16384, 8192] fp32 (1.07 GB)
+// 175 against 165.
+static bool streams(size_t bytes, std::initializer_list<const void *> ptrs)
+{
+    for (const void *p : ptrs)
+        if ((uintptr_t)p & 15) return false;
+    return bytes >= 1000000000;
+}
+
+static bool vec_float(int dt) { return dt == PT_FLOAT32 || dt == PT_FLOAT16 || dt == PT_BFLOAT16; }
+
+// f(integral constant of the dtype) for the vector kernels' types.
+template <typename F>
+static void with_vec_dtype(int dt, F f)
+{
+    if (dt == PT_FLOAT32) f(std::integral_constant<int, PT_FLOAT32>{});
+    else if (dt == PT_FLOAT16) f(std::integral_constant<int, PT_FLOAT16>{});
+    else f(std::integral_constant<int, PT_BFLOAT16>{});
 }
 
 static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t offa,
@@ -565,24 +765,39 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
     hipStream_t st_ = stream_of(stream);
     const char *pa = (const char *)a + offa * dtype_size(dta);
     const char *pb = scalar ? nullptr : (const char *)b + offb * dtype_size(dtb);
-    bool contig = s.ndims <= 1 && (s.ndims == 0 || (s.sa[0] == 1 && (scalar || s.sb[0] == 1)));
-    if (contig && dta == PT_FLOAT32 && (scalar || dtb == PT_FLOAT32) && dto == PT_FLOAT32 &&
-        ((uintptr_t)pa & 15) == 0 && (scalar || ((uintptr_t)pb & 15) == 0) &&
-        ((uintptr_t)out & 15) == 0) {
-        float sv = scalar ? (float)scalar_as_double(scalar) : 0.0f;
-        k_binary_f32_contig<<<grid_for(s.total, 4), 256, 0, st_>>>(
-            (const float *)pa, (const float *)pb, (float *)out, op, s.total, scalar != nullptr, sv, reverse);
-    } else if (!scalar && dta == PT_FLOAT32 && dtb == PT_FLOAT32 && dto == PT_FLOAT32 &&
-               rows_f32(s, pa, pb, out)) {
-        // 2-D row/column broadcasts of float32 (bias adds, row scalings)
-        const unsigned rows = s.ndims == 2 ? (unsigned)s.shape[0] : 1u;
-        const unsigned cols = (unsigned)s.shape[s.ndims - 1];
-        const long long ra = s.ndims == 2 ? s.sa[0] : 0, rb = s.ndims == 2 ? s.sb[0] : 0;
-        const unsigned n4 = rows * (cols / 4);
-        k_binary_f32_rows<<<(n4 + 255) / 256, 256, 0, st_>>>((const float *)pa, (const float *)pb, (float *)out,
-                                                              op, rows, cols / 4, (unsigned)ra,
-                                                              (int)s.sa[s.ndims - 1], (unsigned)rb,
-                                                              (int)s.sb[s.ndims - 1], reverse);
+    Opnd oa, ob;
+    bool vec = vec_float(dta) && (dto == dta || dto == PT_FLOAT32) && (scalar || dtb == dta) &&
+               as_opnd(s, s.sa, pa, oa);
+    if (vec && scalar) ob = Opnd{nullptr, OPND_IMM, 0u, (float)scalar_as_double(scalar)};
+    else vec = vec && as_opnd(s, s.sb, pb, ob);
+    if (vec) {
+        if (reverse) std::swap(oa, ob);
+        const size_t total = (size_t)s.total;
+        const bool nt = streams(total * (dtype_size(dta) * (scalar ? 1 : 2) + dtype_size(dto)),
+                                {oa.mode == OPND_FLAT ? oa.p : nullptr, ob.mode == OPND_FLAT ? ob.p : nullptr, out});
+        with_vec_dtype(dta, [&](auto D) {
+            constexpr int DT = decltype(D)::value;
+            const unsigned grid = grid_for(s.total, 16 / (int)sizeof(typename VecT<DT>::T)), cols = opnd_cols(s);
+            auto go = [&](auto O, auto MA, auto MB) {
+                constexpr int DO = decltype(O)::value, A = decltype(MA)::value, B = decltype(MB)::value;
+                if (nt) k_binary_vec<DT, DO, true, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
+                else k_binary_vec<DT, DO, false, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
+            };
+            // the layouts of most calls have kernels of their own: y * z of
+            // a row and [16384, 8192] fp32 took 181 us with the layouts read
+            // at run time (two branches before the loads) against 169.5
+            // (177 with the contiguous operand loaded before the row)
+            using FL = std::integral_constant<int, OPND_FLAT>;
+            using IM = std::integral_constant<int, OPND_IMM>;
+            using RW = std::integral_constant<int, OPND_ROWS>;
+            using AN = std::integral_constant<int, OPND_ANY>;
+            if (dto != dta) go(std::integral_constant<int, PT_FLOAT32>{}, AN{}, AN{});
+            else if (oa.mode == OPND_FLAT && ob.mode == OPND_FLAT) go(D, FL{}, FL{});
+            else if (oa.mode == OPND_FLAT && ob.mode == OPND_IMM) go(D, FL{}, IM{});
+            else if (oa.mode == OPND_FLAT && ob.mode == OPND_ROWS) go(D, FL{}, RW{});
+            else if (oa.mode == OPND_ROWS && ob.mode == OPND_FLAT) go(D, RW{}, FL{});
+            else go(D, AN{}, AN{});
+        });
     } else {
         EwShape32 s32;
         const bool i32 = to32(s, s32);
@@ -642,15 +857,29 @@ pt_status pt_unary(const void *input, int dtype, const size_t *strides, size_t o
     if (s.total == 0) return PT_OK;
     hipStream_t st_ = stream_of(stream);
     const char *px = (const char *)input + offset * dtype_size(dtype);
-    bool contig = s.ndims <= 1 && (s.ndims == 0 || s.sa[0] == 1);
-    if (contig && dtype == PT_FLOAT32 && ((uintptr_t)px & 15) == 0 && ((uintptr_t)out & 15) == 0) {
-        const unsigned g = grid_for(s.total, 4);
-        if (op == PT_OP_TANH)
-            k_unary_f32_contig<PT_OP_TANH><<<g, 256, 0, st_>>>((const float *)px, (float *)out, op, s.total);
-        else if (op == PT_OP_EXP)
-            k_unary_f32_contig<PT_OP_EXP><<<g, 256, 0, st_>>>((const float *)px, (float *)out, op, s.total);
-        else
-            k_unary_f32_contig<-1><<<g, 256, 0, st_>>>((const float *)px, (float *)out, op, s.total);
+    Opnd ox;
+    if (vec_float(dtype) && as_opnd(s, s.sa, px, ox)) {
+        const size_t total = (size_t)s.total;
+        const bool nt = streams(total * dtype_size(dtype) * 2, {ox.mode == OPND_FLAT ? px : nullptr, out});
+        with_vec_dtype(dtype, [&](auto D) {
+            constexpr int DT = decltype(D)::value;
+            const unsigned grid = grid_for(s.total, 16 / (int)sizeof(typename VecT<DT>::T)), cols = opnd_cols(s);
+            auto go = [&](auto O, auto N) {
+                constexpr int OP = decltype(O)::value;
+                constexpr bool NT = decltype(N)::value;
+                if (ox.mode == OPND_FLAT)
+                    k_unary_vec<DT, OP, NT, OPND_FLAT><<<grid, 256, 0, st_>>>(ox, out, op, total, cols);
+                else
+                    k_unary_vec<DT, OP, NT, OPND_ANY><<<grid, 256, 0, st_>>>(ox, out, op, total, cols);
+            };
+            auto pick = [&](auto N) {
+                if (op == PT_OP_TANH) go(std::integral_constant<int, PT_OP_TANH>{}, N);
+                else if (op == PT_OP_EXP) go(std::integral_constant<int, PT_OP_EXP>{}, N);
+                else go(std::integral_constant<int, -1>{}, N);
+            };
+            if (nt) pick(std::true_type{});
+            else pick(std::false_type{});
+        });
     } else {
         EwShape32 s32;
         const bool i32 = to32(s, s32);
@@ -689,8 +918,23 @@ pt_status pt_cast(const void *input, int dtype_in, const size_t *strides, size_t
                                         hipMemcpyDeviceToDevice, st_), "cast copy"));
         return PT_OK;
     }
+    Opnd ox;
     EwShape32 s32;
-    if (to32(s, s32)) k_cast<EwShape32><<<grid_for(s.total), 256, 0, st_>>>(px, dtype_in, out, dtype_out, s32);
+    if (vec_float(dtype_in) && vec_float(dtype_out) && dtype_in != dtype_out && as_opnd(s, s.sa, px, ox)) {
+        const size_t total = (size_t)s.total;
+        const bool nt = streams(total * (dtype_size(dtype_in) + dtype_size(dtype_out)),
+                                {ox.mode == OPND_FLAT ? px : nullptr, out});
+        with_vec_dtype(dtype_in, [&](auto I) {
+            with_vec_dtype(dtype_out, [&](auto O) {
+                constexpr int DI = decltype(I)::value, DO = decltype(O)::value;
+                if constexpr (DI != DO) {
+                    const unsigned grid = grid_for(s.total, 8);
+                    if (nt) k_cast_vec<DI, DO, true><<<grid, 256, 0, st_>>>(ox, out, total, opnd_cols(s));
+                    else k_cast_vec<DI, DO, false><<<grid, 256, 0, st_>>>(ox, out, total, opnd_cols(s));
+                }
+            });
+        });
+    } else if (to32(s, s32)) k_cast<EwShape32><<<grid_for(s.total), 256, 0, st_>>>(px, dtype_in, out, dtype_out, s32);
     else k_cast<EwShape><<<grid_for(s.total), 256, 0, st_>>>(px, dtype_in, out, dtype_out, s);
     PT_LAUNCH_CHECK("cast");
     counters().elementwise_calls++;
@@ -709,8 +953,34 @@ pt_status pt_where(const void *cond, int dtype_cond, const size_t *strides_cond,
     collapse(shape, ndims, strides_x, strides_y, strides_cond, s);
     if (s.total == 0) return PT_OK;
     hipStream_t st_ = stream_of(stream);
+    Opnd oc, ox, oy;
     EwShape32 s32;
-    if (to32(s, s32))
+    const int csz = (int)dtype_size(dtype_cond), esz = (int)dtype_size(dtype_xy);
+    if (csz <= 4 && (esz == 2 || esz == 4) && as_opnd(s, s.sc, cond, oc) && as_opnd(s, s.sa, x, ox) &&
+        as_opnd(s, s.sb, y, oy)) {
+        const size_t total = (size_t)s.total;
+        // a floating condition holds unless it is +0 or -0; integers and bool unless they are 0
+        const uint32_t mask = dtype_is_floating(dtype_cond) ? (csz == 4 ? 0x7fffffffu : 0x7fffu) : 0xffffffffu;
+        const bool nt = streams(total * (size_t)(csz + 3 * esz),
+                                {oc.mode == OPND_FLAT ? cond : nullptr, ox.mode == OPND_FLAT ? x : nullptr,
+                                 oy.mode == OPND_FLAT ? y : nullptr, out});
+        auto go = [&](auto E, auto C, auto N) {
+            constexpr int ES = decltype(E)::value, CS = decltype(C)::value;
+            k_where_vec<ES, CS, decltype(N)::value><<<grid_for(s.total, 16 / ES), 256, 0, st_>>>(oc, ox, oy, out, mask,
+                                                                                              total, opnd_cols(s));
+        };
+        auto pick = [&](auto E, auto C) {
+            if (nt) go(E, C, std::true_type{});
+            else go(E, C, std::false_type{});
+        };
+        auto by_cond = [&](auto E) {
+            if (csz == 1) pick(E, std::integral_constant<int, 1>{});
+            else if (csz == 2) pick(E, std::integral_constant<int, 2>{});
+            else pick(E, std::integral_constant<int, 4>{});
+        };
+        if (esz == 2) by_cond(std::integral_constant<int, 2>{});
+        else by_cond(std::integral_constant<int, 4>{});
+    } else if (to32(s, s32))
         k_where<EwShape32><<<grid_for(s.total), 256, 0, st_>>>(cond, dtype_cond, x, y, (int)dtype_size(dtype_xy), out,
                                                                s32);
     else
