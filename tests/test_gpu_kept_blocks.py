@@ -1,0 +1,128 @@
+"""Freed blocks kept for the runtime stream's next allocations: a block comes
+back for the same rounded size, never while it is held, never into or out of a
+stream capture, and stays within the bound; threads that share the stream keep
+their values."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+from phptensors import _abi as A
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    L = A.load()
+    A.check(L.pt_init(), "init")
+    yield L
+    A.check(L.pt_mem_init(0), "bound")
+
+
+def _alloc(lib, nbytes, stream=None):
+    p = ctypes.c_void_p()
+    A.check(lib.pt_alloc(ctypes.byref(p), nbytes, stream), "alloc")
+    return p.value
+
+
+@pytest.mark.parametrize("nbytes", [1, 511, 512, 513, 8191, 8192, 8193, 100000, 1 << 20, (1 << 20) + 1, 50_000_001])
+def test_block_returns_for_its_size_only(lib, nbytes):
+    p = _alloc(lib, nbytes)
+    A.check(lib.pt_free(p, None))
+    q = _alloc(lib, nbytes)
+    assert q == p
+    r = _alloc(lib, nbytes)  # p is held: another block
+    assert r != q and abs(r - q) >= nbytes
+    x = np.arange(nbytes % 251 + 1, dtype=np.uint8)[:nbytes]
+    A.check(lib.pt_memcpy_h2d(q, x.ctypes.data, x.nbytes, None))
+    A.check(lib.pt_memset(r, 7, nbytes, None))
+    y = np.empty_like(x)
+    A.check(lib.pt_memcpy_d2h(y.ctypes.data, q, y.nbytes, None))
+    assert np.array_equal(x, y)
+    # bigger than twice the block: never served from it
+    A.check(lib.pt_free(q, None))
+    s = _alloc(lib, 4 * nbytes + 4096)
+    assert s != q
+    for b in (r, s):
+        A.check(lib.pt_free(b, None))
+
+
+def test_other_streams_and_captures_pass_by(lib):
+    """A block freed on another stream is not kept; a capture of the runtime
+    stream neither takes nor gives blocks, and its replays stay right while
+    eager work reuses everything that is kept."""
+    stream = ctypes.c_void_p()
+    A.check(lib.pt_stream_create(ctypes.byref(stream)))
+    p = _alloc(lib, 70000)
+    A.check(lib.pt_stream_synchronize(None))
+    A.check(lib.pt_free(p, stream))
+    q = _alloc(lib, 70000)
+    A.check(lib.pt_free(q, None))
+    A.check(lib.pt_stream_synchronize(stream))
+    A.check(lib.pt_stream_destroy(stream))
+
+    rng = np.random.default_rng(3)
+    x = np.round(rng.uniform(-8, 8, (9000, 40))).astype(np.float32)
+    dx, out = A.to_device(x), A.DeviceBuffer(160)
+    shape, strides = A.ints(x.shape), A.sizes([40, 1])
+    op = A.OP["sum"]
+
+    def reduce():  # splits the rows: its scratch comes from the pool, or from the graph
+        A.check(lib.pt_reduce(dx.ptr, out.ptr, A.FLOAT32, op, shape, strides, 2, 0, 0, None), "sum")
+
+    reduce()
+    graph = ctypes.c_void_p()
+    A.check(lib.pt_graph_begin_capture(None))
+    reduce()
+    A.check(lib.pt_graph_end_capture(None, ctypes.byref(graph)))
+    for i in range(6):
+        A.check(lib.pt_memset(out.ptr, 0xFF, 160, None))
+        A.check(lib.pt_graph_launch(graph, None))
+        junk = [A.DeviceBuffer(n) for n in (40 * 128 * 4, 20480, 512, 100000)]
+        for j in junk:
+            A.check(lib.pt_memset(j.ptr, 0xFF, j.nbytes, None))
+        assert np.array_equal(out.download(np.float32, (40,)), x.sum(0)), i
+        for j in junk:
+            j.free()
+    A.check(lib.pt_graph_destroy(graph))
+
+
+def test_bound(lib):
+    """Blocks beyond the bound go back to the driver's pool, and the bound can be lowered."""
+    A.check(lib.pt_mem_init(1 << 20))
+    blocks = [_alloc(lib, 300_000) for _ in range(8)]
+    for b in blocks:
+        A.check(lib.pt_free(b, None))
+    big = _alloc(lib, 8 << 20)  # larger than the bound: not kept
+    A.check(lib.pt_free(big, None))
+    again = [_alloc(lib, 300_000) for _ in range(8)]
+    assert len(set(again)) == 8
+    for b in again:
+        A.check(lib.pt_free(b, None))
+    A.check(lib.pt_mem_init(0))
+
+
+def test_threads_share_the_stream(lib):
+    from phptensors import CudaArray
+    errors = []
+
+    def work(k):
+        try:
+            for i in range(200):
+                n = 1000 + 37 * ((i + k) % 5)
+                a = CudaArray.full([n], float(k + 1))
+                b = a * 3.0 + a
+                if i % 20 == 0 and not np.all(b.toNumpy() == 4.0 * (k + 1)):
+                    errors.append((k, i))
+                del a, b
+        except Exception as exc:  # reported by the main thread
+            errors.append((k, repr(exc)))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not any(t.is_alive() for t in threads) and not errors, errors[:3]
