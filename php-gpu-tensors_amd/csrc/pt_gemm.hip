@@ -864,8 +864,8 @@ static void launch_dt(GemmArgs g, int tile, bool a_kc, bool b_kc, bool check, hi
         if constexpr (DT == PT_FLOAT32) launch_layouts<DT, 128, 64, 2 * BK, 2, 2, 2>(g, a_kc, b_kc, check, s);
         break;
     case TILE_F32_RING:
-        // fp32 operands in 16-byte packs with whole K steps run the ring
-        // kernel (edge tiles included); others the 8-wave 128x128 kernel
+        // fp32 operands in 16-byte packs run the ring kernel (edge tiles
+        // and K tails included); others the 8-wave 128x128 kernel
         if constexpr (DT == PT_FLOAT32) {
             if (gemm_f32r_eligible(g, a_kc, b_kc)) {
                 launch_gemm_f32r(g, a_kc, b_kc, ring_stages(g.ksplit > 1), s);
@@ -1112,7 +1112,7 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         g.vec_b = vb;
     }
     // fp32 products of 128 x 128 tiles or more run the ring kernel wherever
-    // it takes the operands (16-byte packs, whole 32-k steps); the others
+    // it takes the operands (16-byte packs, any K); the others
     // keep the 256x256 or 8-wave 128x128 tiles chosen above.  Config 4 fp32
     // at steady state: 3711-3721 us against 3913 us (256x256); the config-5
     // products: G2 64.1 us against 73.3 us, dW2 69.8 against 78.0 us.
@@ -1162,6 +1162,7 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         }
     }
     const bool f32ring = dtype == PT_FLOAT32 && tile == TILE_F32_RING && gemm_f32r_eligible(g, a_kc, b_kc);
+    const bool ktail = g.K % 16 != 0;  // the ring's element-wise tail
     switch (dtype) {
     case PT_BFLOAT16: launch_dt<PT_BFLOAT16>(g, tile, a_kc, b_kc, check, s); break;
     case PT_FLOAT16: launch_dt<PT_FLOAT16>(g, tile, a_kc, b_kc, check, s); break;
@@ -1190,14 +1191,14 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         PT_TRY(check_hip(e2, "matmul (split-K sum)"));
         counters().mfma_gemm_calls++;
         snprintf(counters().last_matmul, sizeof(counters().last_matmul), "%s%s",
-                 f32ring ? "mfma-fp32-ring-splitk" : dtype == PT_FLOAT32 ? "mfma-fp32-splitk" : "mfma-low-precision-splitk",
+                 f32ring ? (ktail ? "mfma-fp32-tail-splitk" : "mfma-fp32-ring-splitk") : dtype == PT_FLOAT32 ? "mfma-fp32-splitk" : "mfma-low-precision-splitk",
                  suffix);
         return PT_OK;
     }
     PT_LAUNCH_CHECK("matmul");
     counters().mfma_gemm_calls++;
     snprintf(counters().last_matmul, sizeof(counters().last_matmul), "%s%s",
-             f32ring ? "mfma-fp32-ring" : dtype == PT_FLOAT32 ? "mfma-fp32" : "mfma-low-precision", suffix);
+             f32ring ? (ktail ? "mfma-fp32-tail" : "mfma-fp32-ring") : dtype == PT_FLOAT32 ? "mfma-fp32" : "mfma-low-precision", suffix);
     return PT_OK;
 }
 

@@ -48,10 +48,12 @@ namespace pt {
 //     workgroup's waves keep the SIMD busy while these wait.
 // Fragments of slice s + 1 are read while slice s runs on the matrix cores.
 // Edge tiles: rows past M (columns past N) load the last whole row or
-// 16-byte pack instead and are not stored.  K must be a multiple of 16: a K
-// chunk that ends half-way through its last 32-k step reads that step's
-// loads within the operand's extent (the buffer resource's range) and zeroes
-// both operands' fragments of its last two 8-k slices.
+// 16-byte pack instead and are not stored.  A K chunk that ends within its
+// last 32-k step (TAIL) reads that step's loads within the operand's extent
+// (the buffer resource's range) and zeroes both operands' fragment elements
+// past its end.  4000 x 1024 x 1000 (both operands k-contiguous): 77 us,
+// against 93 us on the 8-wave k_gemm that a K of no multiple of 16 ran
+// before.
 template <bool A_KC, bool B_KC, int NST, bool TAIL>
 __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void k_gemm_f32r(GemmArgs g)
 {
@@ -126,16 +128,15 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void k_gemm_f32r(GemmArgs g)
     const char *B0 = (const char *)(B + (B_KC ? (long long)n0 * g.b_sn : (long long)n0));
     const long long sta = (A_KC ? (long long)BK : (long long)BK * g.a_sk) * 4;
     const long long stb = (B_KC ? (long long)BK : (long long)BK * g.b_sk) * 4;
-    // a K chunk may end half-way through its last 32-k step (K a multiple
-    // of 16): that step's loads reach 16 k past the chunk, and the loads of
-    // each step may read only up to the operand's last element (the buffer
-    // unit returns zeros past it)
+    // a K chunk may end within its last 32-k step: that step's loads reach
+    // past the chunk, and the loads of each step may read only up to the
+    // operand's last element (the buffer unit returns zeros past it)
     const int KT = (Kl + BK - 1) / BK;
-    // TAIL (K not a multiple of 32): the step whose upper half lies past
-    // the chunk (-1: none), compared as a uniform integer so that the check
+    // TAIL (K not a multiple of 32): the step that ends past the chunk (-1:
+    // none), compared as a uniform integer so that the check
     // stays a scalar branch.  Without TAIL the kernel has neither this check
     // nor the range limit, which cost its loop 1.1 % on 4096 x 1024 x 4096.
-    const int half_step = TAIL && (Kl % BK) != 0 ? KT - 1 : -1;
+    const int tail_step = TAIL && (Kl % BK) != 0 ? KT - 1 : -1;
     const char *endA = (const char *)((const float *)g.a + oa +
                                       (long long)(g.M - 1) * g.a_sm + (long long)(g.K - 1) * g.a_sk + 1);
     const char *endB = (const char *)((const float *)g.b + ob +
@@ -251,18 +252,20 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void k_gemm_f32r(GemmArgs g)
     // slices 0-2, the loads of step kt + 3
     auto slice = [&](int kt, auto J, auto S) {
         constexpr int j = decltype(J)::value, s = decltype(S)::value, st = s & 1;
-        if constexpr (TAIL && s >= 2) {
-            // k 16..31 of a half step past the chunk's end: both operands'
-            // fragments are zeroed, so these MFMAs add exact zeros whatever
-            // the loads brought (the next row's values, or zeros)
-            if (kt == half_step) {
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    if constexpr (A_KC) fak[st][i] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (B_KC) fbk[st][i] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
-                }
+        if constexpr (TAIL) {
+            // elements past the chunk's end are zeroed in both operands, so
+            // that their MFMAs add exact zeros whatever the loads brought
+            // (the next row's values, or zeros)
+            if (kt == tail_step) {
+                const int left = Kl - (kt * BK + 8 * s + 4 * (lane >> 5));  // this lane's k from here to the end
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
+                    if (e < left) continue;
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        if constexpr (A_KC) fak[st][i][e] = 0.0f;
+                        if constexpr (B_KC) fbk[st][i][e] = 0.0f;
+                    }
                     if constexpr (!A_KC) fam[st][e] = (f32x2v_t){0.0f, 0.0f};
                     if constexpr (!B_KC) fbm[st][e] = (f32x2v_t){0.0f, 0.0f};
                 }
@@ -347,12 +350,11 @@ bool gemm_f32r_eligible(const GemmArgs &g, bool a_kc, bool b_kc)
 {
     // 16-byte packs along each operand's contiguous dimension (vec_a /
     // vec_b: contiguous stride 1, pitch and batch offsets multiples of 4,
-    // aligned base), K a multiple of 16 (a last half step of 32 is
-    // zero-filled; split chunks are whole steps), for an m- or n-contiguous operand a
-    // whole last pack to clamp edge loads to, and pitches that keep a lane's
+    // aligned base; the last of split chunks may end within a step), for an
+    // m- or n-contiguous operand a whole last pack to clamp edge loads to, and pitches that keep a lane's
     // byte offset within a step (at most 127 pitches) in 32 bits
     constexpr long long kMaxPitch = 1LL << 22;
-    return g.vec_a && g.vec_b && g.K % 16 == 0 && (g.ksplit <= 1 || g.k_chunk % 32 == 0) &&
+    return g.vec_a && g.vec_b && (g.ksplit <= 1 || g.k_chunk % 32 == 0) &&
            (a_kc ? (g.a_sk == 1 && g.a_sm <= kMaxPitch) : (g.a_sm == 1 && g.a_sk <= kMaxPitch && g.M % 4 == 0 && g.M >= 4)) &&
            (b_kc ? (g.b_sk == 1 && g.b_sn <= kMaxPitch) : (g.b_sn == 1 && g.b_sk <= kMaxPitch && g.N % 4 == 0 && g.N >= 4));
 }
@@ -371,7 +373,7 @@ void launch_gemm_f32r(const GemmArgs &g, bool a_kc, bool b_kc, int stages, hipSt
             else k_gemm_f32r<false, false, NST, TAIL><<<grid, 256, 0, s>>>(g);
         }
     };
-    // a K that ends half-way through a 32-k step runs the 4-stage tail form
+    // a K that ends within a 32-k step runs the 4-stage tail form
     if (g.K % 32 != 0) go(IC<4>{}, IC<1>{});
     else if (stages == 2) go(IC<2>{}, IC<0>{});
     else go(IC<4>{}, IC<0>{});
