@@ -29,7 +29,8 @@ struct GemmArgs {
     long long bsa[GEMM_MAX_BATCH_DIMS];
     long long bsb[GEMM_MAX_BATCH_DIMS];
     int remap;             // total tiles divisible by 8: XCD remap on
-    int vec_a, vec_b;      // 16-byte aligned packs: the checked kernel loads in-range packs whole
+    int vec_a, vec_b;      // 16-byte packs along the contiguous dimension, all aligned
+    int con_a, con_b;      // contiguous along one dimension, any alignment
     int ksplit, k_chunk;   // split-K: blockIdx.y = K chunk of k_chunk (a multiple of BK)
     float *partial;        // split-K fp32 partials [ksplit][batch][M][N]
 };

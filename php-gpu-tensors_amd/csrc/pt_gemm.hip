@@ -37,8 +37,12 @@
 
 namespace pt {
 
-// 16-byte pack type for register staging.
+// 16-byte pack type for register staging; GPack: as it lies in memory, at
+// any element (gfx950 loads 16 bytes from every address).
 typedef uint32_t Pack __attribute__((ext_vector_type(4)));
+typedef uint32_t GPack __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t GHalf __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t GWord __attribute__((aligned(2)));
 
 // Gather PK k rows of VR consecutive r elements (raw[k][dword]) and emit VR
 // k-contiguous packs.
@@ -67,7 +71,7 @@ __device__ __forceinline__ void transpose_to_packs(const uint32_t (&raw)[GE<DT>:
     }
 }
 
-template <int DT, int BM, int BN, int BK, int WM, int WN, bool A_KC, bool B_KC, bool CHECK>
+template <int DT, int BM, int BN, int BK, int WM, int WN, bool A_KC, bool B_KC>
 struct GemmCfg {
     using S = typename GE<DT>::S;
     static constexpr int PK = GE<DT>::PK;
@@ -97,22 +101,53 @@ __device__ __forceinline__ S load_elem_checked(const S *p, long long off, bool o
     return ok ? p[off] : (S)0;
 }
 
+// `w` (N dwords of packed elements) moved down by `n` elements of S.
+template <typename S, int N>
+__device__ __forceinline__ void shift_down(uint32_t (&w)[N], int n)
+{
+    constexpr int EPW = 4 / (int)sizeof(S);
+    if constexpr (EPW == 2) {
+        const bool odd = n & 1;
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const uint32_t hi = q + 1 < N ? w[q + 1] : 0u;
+            w[q] = odd ? (w[q] >> 16) | (hi << 16) : w[q];
+        }
+    }
+    // whole dwords, by 2 and by 1
+    const int d = n / EPW;
+#pragma unroll
+    for (int q = 0; q < N; q++) w[q] = (d & 2) ? (q + 2 < N ? w[q + 2] : 0u) : w[q];
+#pragma unroll
+    for (int q = 0; q < N; q++) w[q] = (d & 1) ? (q + 1 < N ? w[q + 1] : 0u) : w[q];
+}
+
+// How a tile is staged: LOAD_PLAIN, whole tiles inside the matrix; LOAD_EDGE,
+// packs moved back into the matrix at its edges; LOAD_CHECK, every element
+// tested.
+enum { LOAD_PLAIN = 0, LOAD_EDGE, LOAD_CHECK };
+
 // Stage one operand tile (R rows x BK k) from global memory into registers.
 // KC: k is the contiguous dimension of the source.  KM (r-contiguous
 // sources only): the tile goes to LDS k-major, [k][r], as 16-byte packs of
 // r loaded and stored whole; fragment reads then gather their k values.
-template <int DT, int R, int BK, int T, bool KC, bool CHECK, bool KM = false, bool CLAMP = false>
+// LOAD_EDGE: rows past r_total read the last row instead (they only feed
+// outputs that are not stored); a pack of r that would straddle r_total is
+// loaded where it ends with the matrix and moved down to its place.  A K
+// that ends within a step loads that step BK back from the end (`k0`) and
+// zeroes, in both operands, the `kskip` k that the step before it had, so
+// that every load is whole and no sum holds an element twice.
+template <int DT, int R, int BK, int T, bool KC, int MODE, bool KM = false>
 struct TileLoader {
     using S = typename GE<DT>::S;
     static constexpr int PK = GE<DT>::PK;
     static constexpr int P = R * BK / PK / T;         // packs per thread (KC, KM)
     static constexpr int VR = R * BK / (T * PK);      // r per thread (RC)
     static constexpr int DW = (VR * (int)sizeof(S) + 3) / 4;  // dwords per RC row load
+    static constexpr bool CHECK = MODE == LOAD_CHECK, EDGE = MODE == LOAD_EDGE;
+    // elements of r that one load takes
+    static constexpr int RL = KC ? 1 : KM ? PK : VR;
     static_assert(!KM || (!KC && P >= 1 && (R / PK) * BK % T == 0), "k-major staging");
-    // CLAMP (unchecked loads on an edge tile): rows past r_total read the
-    // last whole row or pack instead; they only feed outputs that are not
-    // stored
-    static_assert(!CLAMP || (!CHECK && (KC || KM)), "clamped staging");
     Pack kc[(KC || KM) ? P : 1];
     uint32_t rc[(KC || KM) ? 1 : PK][(KC || KM) ? 1 : (DW > 0 ? DW : 1)];
 
@@ -121,6 +156,7 @@ struct TileLoader {
     __device__ __forceinline__ void load(const S *base, long long s_r, long long s_k, int r0,
                                          int r_total, int k0, int K, int tid, int vec = 0)
     {
+        const bool moves = EDGE && r0 + R > r_total;  // a load may straddle r_total (uniform)
         if constexpr (KM) {
             // pack p: k row p / (R / PK), r pack p % (R / PK); a wave reads
             // whole rows of r
@@ -129,9 +165,14 @@ struct TileLoader {
                 int p = tid + j * T;
                 int k = p / (R / PK), rp = p % (R / PK);
                 int gr = r0 + rp * PK, gk = k0 + k;
-                if constexpr (CLAMP) gr = min(gr, r_total - PK);
                 if (!CHECK || (vec && gk < K && gr + PK <= r_total)) {
-                    kc[j] = *(const Pack *)(base + (long long)gk * s_k + gr);
+                    const int at = EDGE ? min(gr, r_total - PK) : gr;
+                    kc[j] = *(const GPack *)(base + (long long)gk * s_k + at);
+                    if (moves) {
+                        uint32_t w[4] = {kc[j][0], kc[j][1], kc[j][2], kc[j][3]};
+                        shift_down<S>(w, min(gr - at, PK - 1));
+                        kc[j] = (Pack){w[0], w[1], w[2], w[3]};
+                    }
                 } else {
                     Pack pk = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -149,9 +190,9 @@ struct TileLoader {
                 int p = tid + j * T;
                 int r = p / (BK / PK), kp = p % (BK / PK);
                 int gr = r0 + r, gk = k0 + kp * PK;
-                if constexpr (CLAMP) gr = min(gr, r_total - 1);
+                if constexpr (EDGE) gr = min(gr, r_total - 1);
                 if (!CHECK || (vec && gr < r_total && gk + PK <= K)) {
-                    kc[j] = *(const Pack *)(base + (long long)gr * s_r + gk);
+                    kc[j] = *(const GPack *)(base + (long long)gr * s_r + gk);
                 } else {
                     Pack pk = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -171,18 +212,20 @@ struct TileLoader {
             for (int e = 0; e < PK; e++) {
                 int gk = k0 + kg * PK + e;
                 if (!CHECK || (vec && gk < K && gr + VR <= r_total)) {
-                    const S *p = base + (long long)gk * s_k + gr;
+                    const int at = EDGE ? min(gr, r_total - VR) : gr;
+                    const S *p = base + (long long)gk * s_k + at;
                     if constexpr (VR * sizeof(S) == 16) {
-                        uint4 v = *(const uint4 *)p;
+                        const GPack v = *(const GPack *)p;
                         rc[e][0] = v.x; rc[e][1] = v.y; rc[e][2] = v.z; rc[e][3] = v.w;
                     } else if constexpr (VR * sizeof(S) == 8) {
-                        uint2 v = *(const uint2 *)p;
+                        const GHalf v = *(const GHalf *)p;
                         rc[e][0] = v.x; rc[e][1] = v.y;
                     } else if constexpr (VR * sizeof(S) == 4) {
-                        rc[e][0] = *(const uint32_t *)p;
+                        rc[e][0] = *(const GWord *)p;
                     } else {
                         rc[e][0] = *(const uint16_t *)p;
                     }
+                    if (VR > 1 && moves) shift_down<S>(rc[e], min(gr - at, VR - 1));
                 } else {
 #pragma unroll
                     for (int q = 0; q < DW; q++) rc[e][q] = 0u;
@@ -194,6 +237,37 @@ struct TileLoader {
                     }
                 }
             }
+        }
+    }
+
+    // Zero the staged elements of the step's first `kskip` k.
+    __device__ __forceinline__ void skip(int kskip, int tid)
+    {
+        if constexpr (KM) {
+#pragma unroll
+            for (int j = 0; j < P; j++)
+                if ((tid + j * T) / (R / PK) < kskip) kc[j] = (Pack){0u, 0u, 0u, 0u};
+        } else if constexpr (KC) {
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                const int n = kskip - (tid + j * T) % (BK / PK) * PK;  // of this pack's elements
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if constexpr (sizeof(S) == 4) {
+                        if (q < n) kc[j][q] = 0u;
+                    } else {
+                        if (2 * q + 1 < n) kc[j][q] = 0u;
+                        else if (2 * q < n) kc[j][q] &= 0xffff0000u;
+                    }
+                }
+            }
+        } else {
+            const int kg = tid / (R / VR);
+#pragma unroll
+            for (int e = 0; e < PK; e++)
+                if (kg * PK + e < kskip)
+#pragma unroll
+                    for (int q = 0; q < DW; q++) rc[e][q] = 0u;
         }
     }
 
@@ -243,15 +317,14 @@ struct GemmLds {
     static constexpr int SB = BKM ? BK * LDB : BN * LDK;
 };
 
-template <int DT, int BM, int BN, int BK, int WM, int WN, bool A_KC, bool B_KC, bool CHECK, int SCHED,
-          bool CLAMP = false>
+template <int DT, int BM, int BN, int BK, int WM, int WN, bool A_KC, bool B_KC, int MODE, int SCHED>
 __device__ __forceinline__ void gemm_core(const GemmArgs &g,
                                           typename GE<DT>::S (&lds_a)[2][GemmLds<DT, BM, BN, BK, A_KC, B_KC>::SA],
                                           typename GE<DT>::S (&lds_b)[2][GemmLds<DT, BM, BN, BK, A_KC, B_KC>::SB],
                                           const typename GE<DT>::S *A, const typename GE<DT>::S *B, int Kl,
                                           int bidx, int split, int m0, int n0)
 {
-    using C = GemmCfg<DT, BM, BN, BK, WM, WN, A_KC, B_KC, CHECK>;
+    using C = GemmCfg<DT, BM, BN, BK, WM, WN, A_KC, B_KC>;
     using S = typename C::S;
     using L = GemmLds<DT, BM, BN, BK, A_KC, B_KC>;
     constexpr int T = C::T, PK = C::PK, LDK = C::LDK, TM = C::TM, TN = C::TN;
@@ -264,8 +337,8 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
     // Two register staging sets: the global loads of tile k+2 are issued
     // while tile k runs on the matrix cores and tile k+1 waits in the other
     // set, giving the loads two K steps of MFMA work to arrive.
-    using LoaderA = TileLoader<DT, BM, BK, T, A_KC, CHECK, AKM, CLAMP>;
-    using LoaderB = TileLoader<DT, BN, BK, T, B_KC, CHECK, BKM, CLAMP>;
+    using LoaderA = TileLoader<DT, BM, BK, T, A_KC, MODE, AKM>;
+    using LoaderB = TileLoader<DT, BN, BK, T, B_KC, MODE, BKM>;
     LoaderA la[2];
     LoaderB lb[2];
 
@@ -283,10 +356,15 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
     // compiler knows exactly which loads are in flight, and waits for the
     // staged step only, never for the one issued after it.
     // A(m, k): r = m, s_r = a_sm, s_k = a_sk.  B(k, n): r = n, s_r = b_sn, s_k = b_sk.
-    la[0].load(A, g.a_sm, g.a_sk, m0, g.M, 0, Kl, tid, g.vec_a);
-    lb[0].load(B, g.b_sn, g.b_sk, n0, g.N, 0, Kl, tid, g.vec_b);
-    la[1].load(A, g.a_sm, g.a_sk, m0, g.M, min(1, KT - 1) * BK, Kl, tid, g.vec_a);
-    lb[1].load(B, g.b_sn, g.b_sk, n0, g.N, min(1, KT - 1) * BK, Kl, tid, g.vec_b);
+    // LOAD_EDGE (Kl >= BK): the last step of a K that is no multiple of BK
+    // starts at Kl - BK and drops the kskip k it shares with the step before
+    const int klast = MODE == LOAD_EDGE ? Kl - BK : (KT - 1) * BK;
+    const int kskip = MODE == LOAD_EDGE ? KT * BK - Kl : 0;
+    auto k_of = [&](int kt) { return kt < KT - 1 ? kt * BK : klast; };
+    la[0].load(A, g.a_sm, g.a_sk, m0, g.M, k_of(0), Kl, tid, g.con_a);
+    lb[0].load(B, g.b_sn, g.b_sk, n0, g.N, k_of(0), Kl, tid, g.con_b);
+    la[1].load(A, g.a_sm, g.a_sk, m0, g.M, k_of(1), Kl, tid, g.con_a);
+    lb[1].load(B, g.b_sn, g.b_sk, n0, g.N, k_of(1), Kl, tid, g.con_b);
     la[0].template store<LDA>(lds_a[0], tid);
     lb[0].template store<LDB>(lds_b[0], tid);
     __syncthreads();
@@ -350,9 +428,9 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
     // step kt: W holds tile kt+1 (to LDS after the MFMAs), L receives tile kt+2
     auto step = [&](int kt, LoaderA &wa, LoaderB &wb, LoaderA &la_, LoaderB &lb_) {
         const int cur = kt & 1;
-        const int kload = min(kt + 2, KT - 1) * BK;
-        la_.load(A, g.a_sm, g.a_sk, m0, g.M, kload, Kl, tid, g.vec_a);
-        lb_.load(B, g.b_sn, g.b_sk, n0, g.N, kload, Kl, tid, g.vec_b);
+        const int kload = k_of(kt + 2);
+        la_.load(A, g.a_sm, g.a_sk, m0, g.M, kload, Kl, tid, g.con_a);
+        lb_.load(B, g.b_sn, g.b_sk, n0, g.N, kload, Kl, tid, g.con_b);
 #pragma unroll
         for (int sl = 0; sl < NS; sl++) {
             if (sl + 1 < NS)
@@ -374,6 +452,12 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
             }
         }
         // the last step stores and reads a re-read copy that no MFMA uses
+        if constexpr (MODE == LOAD_EDGE) {
+            if (kskip && kt + 1 == KT - 1) {  // (KT > 1: Kl >= BK leaves nothing to drop in the only step)
+                wa.skip(kskip, tid);
+                wb.skip(kskip, tid);
+            }
+        }
         wa.template store<LDA>(lds_a[cur ^ 1], tid);
         wb.template store<LDB>(lds_b[cur ^ 1], tid);
         __syncthreads();
@@ -400,7 +484,7 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
             for (int e = 0; e < 16; e++) {
                 const int rho = (e >> 2) * 8 + row_l + (e & 3);  // row within the 32x32 block
                 const int m = m0 + wm * C::WTM + (AIL ? TM * rho + i : i * 32 + rho);
-                if ((!CHECK && !CLAMP) || (m < g.M && n < g.N)) {
+                if (MODE == LOAD_PLAIN || (m < g.M && n < g.N)) {
                     if (Pb) Pb[(size_t)m * g.N + n] = acc[i][j][e];
                     else store_c<DT>(Cb, (size_t)m * g.N + n, acc[i][j][e]);
                 }
@@ -447,24 +531,28 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm(GemmArgs g)
     const S *B = (const S *)g.b + ob + (long long)kbase * g.b_sk;
 
     if constexpr (CHECK) {
-        // Whole K steps and packable operands: tiles wholly inside M x N run
-        // the unchecked core, edge tiles the same core with clamped rows and
-        // a guarded store (all of one launch's workgroups run at once, so an
-        // edge tile as slow as a checked one would set the launch's time);
-        // only ragged K or unpackable operands pay for per-element checks.
-        constexpr bool CLAMPABLE = (A_KC || L::AKM) && (B_KC || L::BKM);
-        const bool whole = g.vec_a && g.vec_b && Kl % BK == 0;
-        const bool interior = whole && m0 + BM <= g.M && n0 + BN <= g.N;
-        const bool clampable = whole && (A_KC || g.M % GE<DT>::PK == 0) && (B_KC || g.N % GE<DT>::PK == 0);
-        if (interior)
-            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, false, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0, n0);
-        else if (CLAMPABLE && clampable)
-            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, false, SCHED, CLAMPABLE>(g, lds_a, lds_b, A, B, Kl, bidx,
-                                                                                split, m0, n0);
+        // Operands contiguous along one dimension: tiles wholly inside
+        // M x N with whole K steps run the plain core, the others the edge
+        // core, whose loads are as wide (all of one launch's workgroups run
+        // at once, so an edge tile as slow as a checked one would set the
+        // launch's time); only a K or an extent below one load's, and
+        // operands strided in both dimensions, pay for per-element checks.
+        // 12 x 1000 x 1001 x 777 fp16, whose rows are no multiple of 16 bytes:
+        // 47 us, 277 us with every element checked.
+        using LA = TileLoader<DT, BM, BK, 64 * WM * WN, A_KC, LOAD_EDGE, L::AKM>;
+        using LB = TileLoader<DT, BN, BK, 64 * WM * WN, B_KC, LOAD_EDGE, L::BKM>;
+        const bool packs = g.con_a && g.con_b;
+        if (packs && Kl % BK == 0 && m0 + BM <= g.M && n0 + BN <= g.N)
+            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_PLAIN, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0,
+                                                                            n0);
+        else if (packs && Kl >= BK && g.M >= LA::RL && g.N >= LB::RL)
+            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_EDGE, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0,
+                                                                           n0);
         else
-            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, true, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0, n0);
+            gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_CHECK, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0,
+                                                                            n0);
     } else {
-        gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, false, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0, n0);
+        gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_PLAIN, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0, n0);
     }
 }
 
@@ -1098,9 +1186,9 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         }
         tile = TILE_256x256;
     }
-    // checked kernels still load whole 16-byte packs that lie inside the
-    // matrix when the operand's contiguous stride is 1 and its pitch and
-    // batch offsets keep packs aligned
+    // con: the operand's contiguous stride is 1 (the kernels load 16 bytes
+    // from any element); vec: and its base, pitch and batch offsets keep
+    // 16-byte packs aligned
     {
         bool va = aligned(a) && (a_kc ? (g.a_sk == 1 && g.a_sm % PKe == 0) : (g.a_sm == 1 && g.a_sk % PKe == 0));
         bool vb = aligned(b) && (b_kc ? (g.b_sk == 1 && g.b_sn % PKe == 0) : (g.b_sn == 1 && g.b_sk % PKe == 0));
@@ -1110,6 +1198,8 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         }
         g.vec_a = va;
         g.vec_b = vb;
+        g.con_a = a_kc ? g.a_sk == 1 : g.a_sm == 1;
+        g.con_b = b_kc ? g.b_sk == 1 : g.b_sn == 1;
     }
     // fp32 products of 128 x 128 tiles or more run the ring kernel wherever
     // it takes the operands (16-byte packs, any K); the others
