@@ -133,10 +133,11 @@ enum { LOAD_PLAIN = 0, LOAD_EDGE, LOAD_CHECK };
 // r loaded and stored whole; fragment reads then gather their k values.
 // LOAD_EDGE: rows past r_total read the last row instead (they only feed
 // outputs that are not stored); a pack of r that would straddle r_total is
-// loaded where it ends with the matrix and moved down to its place.  A K
-// that ends within a step loads that step BK back from the end (`k0`) and
-// zeroes, in both operands, the `kskip` k that the step before it had, so
-// that every load is whole and no sum holds an element twice.
+// loaded where it ends with the matrix and moved down to its place.  In a
+// step that K ends within, packs of k past the end are loaded where they end
+// with K and rows of k past it re-read the last one; tail() then moves what
+// belongs to the step to its place and zeroes the rest, so that every sum
+// has the order it has with every element tested.
 template <int DT, int R, int BK, int T, bool KC, int MODE, bool KM = false>
 struct TileLoader {
     using S = typename GE<DT>::S;
@@ -167,6 +168,7 @@ struct TileLoader {
                 int gr = r0 + rp * PK, gk = k0 + k;
                 if (!CHECK || (vec && gk < K && gr + PK <= r_total)) {
                     const int at = EDGE ? min(gr, r_total - PK) : gr;
+                    if constexpr (EDGE) gk = min(gk, K - 1);
                     kc[j] = *(const GPack *)(base + (long long)gk * s_k + at);
                     if (moves) {
                         uint32_t w[4] = {kc[j][0], kc[j][1], kc[j][2], kc[j][3]};
@@ -190,7 +192,10 @@ struct TileLoader {
                 int p = tid + j * T;
                 int r = p / (BK / PK), kp = p % (BK / PK);
                 int gr = r0 + r, gk = k0 + kp * PK;
-                if constexpr (EDGE) gr = min(gr, r_total - 1);
+                if constexpr (EDGE) {
+                    gr = min(gr, r_total - 1);
+                    gk = min(gk, K - PK);
+                }
                 if (!CHECK || (vec && gr < r_total && gk + PK <= K)) {
                     kc[j] = *(const GPack *)(base + (long long)gr * s_r + gk);
                 } else {
@@ -213,6 +218,7 @@ struct TileLoader {
                 int gk = k0 + kg * PK + e;
                 if (!CHECK || (vec && gk < K && gr + VR <= r_total)) {
                     const int at = EDGE ? min(gr, r_total - VR) : gr;
+                    if constexpr (EDGE) gk = min(gk, K - 1);
                     const S *p = base + (long long)gk * s_k + at;
                     if constexpr (VR * sizeof(S) == 16) {
                         const GPack v = *(const GPack *)p;
@@ -240,32 +246,27 @@ struct TileLoader {
         }
     }
 
-    // Zero the staged elements of the step's first `kskip` k.
-    __device__ __forceinline__ void skip(int kskip, int tid)
+    // LOAD_EDGE, after the loads of a step [k0, k0 + BK) that K ends within.
+    __device__ __forceinline__ void tail(int k0, int K, int tid)
     {
         if constexpr (KM) {
 #pragma unroll
             for (int j = 0; j < P; j++)
-                if ((tid + j * T) / (R / PK) < kskip) kc[j] = (Pack){0u, 0u, 0u, 0u};
+                if (k0 + (tid + j * T) / (R / PK) >= K) kc[j] = (Pack){0u, 0u, 0u, 0u};
         } else if constexpr (KC) {
 #pragma unroll
             for (int j = 0; j < P; j++) {
-                const int n = kskip - (tid + j * T) % (BK / PK) * PK;  // of this pack's elements
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    if constexpr (sizeof(S) == 4) {
-                        if (q < n) kc[j][q] = 0u;
-                    } else {
-                        if (2 * q + 1 < n) kc[j][q] = 0u;
-                        else if (2 * q < n) kc[j][q] &= 0xffff0000u;
-                    }
-                }
+                const int gk = k0 + (tid + j * T) % (BK / PK) * PK, n = gk - min(gk, K - PK);
+                uint32_t w[4] = {kc[j][0], kc[j][1], kc[j][2], kc[j][3]};
+                shift_down<S>(w, min(n, PK - 1));
+                kc[j] = (Pack){w[0], w[1], w[2], w[3]};
+                if (n >= PK) kc[j] = (Pack){0u, 0u, 0u, 0u};
             }
         } else {
             const int kg = tid / (R / VR);
 #pragma unroll
             for (int e = 0; e < PK; e++)
-                if (kg * PK + e < kskip)
+                if (k0 + kg * PK + e >= K)
 #pragma unroll
                     for (int q = 0; q < DW; q++) rc[e][q] = 0u;
         }
@@ -356,15 +357,19 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
     // compiler knows exactly which loads are in flight, and waits for the
     // staged step only, never for the one issued after it.
     // A(m, k): r = m, s_r = a_sm, s_k = a_sk.  B(k, n): r = n, s_r = b_sn, s_k = b_sk.
-    // LOAD_EDGE (Kl >= BK): the last step of a K that is no multiple of BK
-    // starts at Kl - BK and drops the kskip k it shares with the step before
-    const int klast = MODE == LOAD_EDGE ? Kl - BK : (KT - 1) * BK;
-    const int kskip = MODE == LOAD_EDGE ? KT * BK - Kl : 0;
-    auto k_of = [&](int kt) { return kt < KT - 1 ? kt * BK : klast; };
+    const int klast = (KT - 1) * BK;
+    const bool ends_within = MODE == LOAD_EDGE && klast + BK > Kl;
+    auto k_of = [&](int kt) { return min(kt * BK, klast); };
     la[0].load(A, g.a_sm, g.a_sk, m0, g.M, k_of(0), Kl, tid, g.con_a);
     lb[0].load(B, g.b_sn, g.b_sk, n0, g.N, k_of(0), Kl, tid, g.con_b);
     la[1].load(A, g.a_sm, g.a_sk, m0, g.M, k_of(1), Kl, tid, g.con_a);
     lb[1].load(B, g.b_sn, g.b_sk, n0, g.N, k_of(1), Kl, tid, g.con_b);
+    if constexpr (MODE == LOAD_EDGE) {
+        if (ends_within && KT == 1) {
+            la[0].tail(klast, Kl, tid);
+            lb[0].tail(klast, Kl, tid);
+        }
+    }
     la[0].template store<LDA>(lds_a[0], tid);
     lb[0].template store<LDB>(lds_b[0], tid);
     __syncthreads();
@@ -453,9 +458,9 @@ __device__ __forceinline__ void gemm_core(const GemmArgs &g,
         }
         // the last step stores and reads a re-read copy that no MFMA uses
         if constexpr (MODE == LOAD_EDGE) {
-            if (kskip && kt + 1 == KT - 1) {  // (KT > 1: Kl >= BK leaves nothing to drop in the only step)
-                wa.skip(kskip, tid);
-                wb.skip(kskip, tid);
+            if (ends_within && kt + 1 == KT - 1) {
+                wa.tail(klast, Kl, tid);
+                wb.tail(klast, Kl, tid);
             }
         }
         wa.template store<LDA>(lds_a[cur ^ 1], tid);
@@ -535,7 +540,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm(GemmArgs g)
         // M x N with whole K steps run the plain core, the others the edge
         // core, whose loads are as wide (all of one launch's workgroups run
         // at once, so an edge tile as slow as a checked one would set the
-        // launch's time); only a K or an extent below one load's, and
+        // launch's time); only a K or an extent below one load's and
         // operands strided in both dimensions, pay for per-element checks.
         // 12 x 1000 x 1001 x 777 fp16, whose rows are no multiple of 16 bytes:
         // 47 us, 277 us with every element checked.
@@ -545,7 +550,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm(GemmArgs g)
         if (packs && Kl % BK == 0 && m0 + BM <= g.M && n0 + BN <= g.N)
             gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_PLAIN, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0,
                                                                             n0);
-        else if (packs && Kl >= BK && g.M >= LA::RL && g.N >= LB::RL)
+        else if (packs && Kl >= GE<DT>::PK && g.M >= LA::RL && g.N >= LB::RL)
             gemm_core<DT, BM, BN, BK, WM, WN, A_KC, B_KC, LOAD_EDGE, SCHED>(g, lds_a, lds_b, A, B, Kl, bidx, split, m0,
                                                                            n0);
         else
@@ -1202,14 +1207,17 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         g.con_b = b_kc ? g.b_sk == 1 : g.b_sn == 1;
     }
     // fp32 products of 128 x 128 tiles or more run the ring kernel wherever
-    // it takes the operands (16-byte packs, any K); the others
+    // it takes the operands (16-byte packs); the others
     // keep the 256x256 or 8-wave 128x128 tiles chosen above.  Config 4 fp32
     // at steady state: 3711-3721 us against 3913 us (256x256); the config-5
     // products: G2 64.1 us against 73.3 us, dW2 69.8 against 78.0 us.
     if (dtype == PT_FLOAT32 && g_tile_override < 0 && !tuned && (tile == TILE_256x256 || tile == TILE_128x128_W8)) {
         GemmArgs whole = g;
         whole.ksplit = 1;
-        if (gemm_f32r_eligible(whole, a_kc, b_kc)) tile = TILE_F32_RING;
+        // (a K of no multiple of 16 only where neither kernel splits it: both
+        // then add in the same order)
+        const long long t128 = ((g.M + 127) / 128) * (long long)((g.N + 127) / 128) * batch;
+        if (gemm_f32r_eligible(whole, a_kc, b_kc) && (g.K % 16 == 0 || g.K < 128 || t128 >= 256)) tile = TILE_F32_RING;
     }
     int bm = kTiles[tile].bm, bn = kTiles[tile].bn;
     const int BK = (dtype == PT_FLOAT32 ? 16 : 32) * kTiles[tile].kmul;
