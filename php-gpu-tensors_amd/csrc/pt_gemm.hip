@@ -542,8 +542,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm(GemmArgs g)
         // at once, so an edge tile as slow as a checked one would set the
         // launch's time); only a K or an extent below one load's and
         // operands strided in both dimensions, pay for per-element checks.
-        // 12 x 1000 x 1001 x 777 fp16, whose rows are no multiple of 16 bytes:
-        // 47 us, 277 us with every element checked.
+        // 12 x 1000 x 1001 x 777 fp16 (4 waves), whose rows are no multiple of
+        // 16 bytes: 47 us, 277 us with every element checked.
         using LA = TileLoader<DT, BM, BK, 64 * WM * WN, A_KC, LOAD_EDGE, L::AKM>;
         using LB = TileLoader<DT, BN, BK, 64 * WM * WN, B_KC, LOAD_EDGE, L::BKM>;
         const bool packs = g.con_a && g.con_b;
@@ -1113,16 +1113,30 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
     const char *suffix = tuned ? "-tuned" : "";
     if (tile < 0) {
         long long t256 = ((g.M + 255) / 256) * (long long)((g.N + 255) / 256) * batch;
-        // mid-size fp32: 128x128 tiles of 8 waves for either layout of B
-        // (dZ2 W2^T of config 5, B k-contiguous: 76-78 us against 82-84 us
-        // for 128x64 tiles at two workgroups per CU)
-        const int mid32 = TILE_128x128_W8;
+        // Mid-size products.  128x128 tiles of 8 waves where they give every
+        // CU one: fp32 for either layout of B (dZ2 W2^T of config 5, B
+        // k-contiguous: 76-78 us against 82-84 us for 128x64 tiles at two
+        // workgroups per CU), 16-bit 12 x 1000 x 1001 x 777 fp16 43.5 us
+        // against 52 us with 4 waves, 2048^3 bf16 34.8 against 37.0.
+        // Fewer tiles split K over the CUs, at the price of fp32 partials
+        // and a sum, which pays only over a long K (there 4 waves stay ahead
+        // for 16 bits); below it 64x64 tiles fill the CUs at once.  64x64
+        // against split 128x128, bf16, us, by K 256 / 512 / 1024 / 2048:
+        // 1024 x 1024 6.8/9.8/13.6/23.5 against 13.5/17.2/21.7/21.9,
+        // 512 x 512 (16 tiles) 13.5 against 17.2 at K 2048.  fp32 keeps the
+        // split (1024 x 1024 9.9/14.6/26.6/56.0 against 18.9/24.4/27.7/40.4):
+        // another order of its sums moves single ReLU decisions of a training
+        // step, whose gradients then differ by more than rounding.
+        const long long t128 = ((g.M + 127) / 128) * (long long)((g.N + 127) / 128) * batch;
+        const bool f32 = dtype == PT_FLOAT32;
+        const bool narrow = !f32 && t128 < 256 && (g.K <= 1024 || (g.K <= 2048 && t128 <= 32));
         tile = (g.M >= 256 && g.N >= 256 && t256 >= 256)
-                   ? (dtype == PT_FLOAT32 ? TILE_256x256
+                   ? (f32 ? TILE_256x256
                       : g.K % 64 != 0 ? TILE_RING_HALF
                       : dtype == PT_BFLOAT16 ? TILE_RING_DEFAULT : TILE_RING_DEFAULT_F16)
-                   : (g.M >= 128 && g.N >= 128) ? (dtype == PT_FLOAT32 ? mid32 : TILE_128x128)
-                                                : TILE_64x64;
+               : g.M < 128 || g.N < 128 || narrow ? TILE_64x64
+               : f32 || t128 >= 256               ? TILE_128x128_W8
+                                                  : TILE_128x128;
     }
     // the fp32-only tiles run the 128x128 kernel for 16-bit operands
     if (dtype != PT_FLOAT32 && (tile == TILE_128x128_W8_K2 || tile == TILE_128x64_W4M2 || tile == TILE_128x64_W4M2_K2 ||
