@@ -239,6 +239,14 @@ pt_status pt_layernorm(const void *input, void *output, int input_dtype, int com
                        size_t rows, size_t n, double eps,
                        const void *gamma, const void *beta, pt_stream_t stream);
 
+/* pt_layernorm_params: pt_layernorm with gamma and beta of param_dtype, the
+ * compute dtype or, for f16/bf16 input computed in float32, the input's: the
+ * kernel widens them as it reads them, so that the host need not cast them
+ * on each call. */
+pt_status pt_layernorm_params(const void *input, void *output, int input_dtype, int compute_dtype,
+                              size_t rows, size_t n, double eps,
+                              const void *gamma, const void *beta, int param_dtype, pt_stream_t stream);
+
 /* ------------------------------------------------------------------ GEMM --
  * Replaces cuda_matmul_launcher (src/backends/cuda/matmul_kernels.h:40-44),
  * cuda_batched_matmul_nd_launcher (:47-51) and

@@ -64,6 +64,11 @@ __device__ __forceinline__ void load_chunk(const typename RT<DT>::S *p, typename
         else u.raw = *(const u32x4 *)p;
 #pragma unroll
         for (int i = 0; i < V; i++) v[i] = RT<DT>::cv(u.s[i]);
+    } else if constexpr (V * sizeof(S) == 4) {
+        union { uint32_t raw; S s[V]; } u;
+        memcpy(&u.raw, p, 4);
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] = RT<DT>::cv(u.s[i]);
     } else {
 #pragma unroll
         for (int i = 0; i < V; i++) v[i] = RT<DT>::cv(p[i]);
@@ -949,20 +954,35 @@ __device__ __forceinline__ void load_vec16(const T *p, T (&v)[VEC])
     for (int k = 0; k < VEC; k++) v[k] = u.t[k];
 }
 
+// VEC layerNorm parameters of type PDT.
+template <int PDT, int VEC, typename CT>
+__device__ __forceinline__ void load_params(const typename RT<PDT>::S *p, CT (&v)[VEC])
+{
+    typename RT<PDT>::S t[VEC];
+    load_vec16<typename RT<PDT>::S, VEC>(p, t);
+#pragma unroll
+    for (int k = 0; k < VEC; k++) v[k] = (CT)RT<PDT>::cv(t[k]);
+}
+
 // Fused layerNorm (cuda_array_ce.c:2295-2323): mean, centered, biased
 // variance of the centered values, eps inside the sqrt, true division, then
 // gamma and beta (contiguous [n] arrays).  With WPR = 4 a block walks the
 // rows blockIdx.x, blockIdx.x + gridDim.x, ... and keeps its gamma / beta
 // chunks in registers across them, so they are read once per block instead
 // of once per row.
-template <int DT, int VEC, int NCH, int WPR, typename CT, bool FULL = false, bool LNT = false, bool SNT = false>
+// PDT: the parameters' type, CT's or a 16-bit input's (widened as they are
+// read, the values a cast before the call would give).
+template <int DT, int VEC, int NCH, int WPR, typename CT, int PDT, bool FULL = false, bool LNT = false,
+          bool SNT = false>
 __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_layernorm(const void *__restrict__ xin, size_t rows,
                                                                            int n, CT eps,
-                                                                           const CT *__restrict__ gamma,
-                                                                           const CT *__restrict__ beta,
+                                                                           const void *__restrict__ gamma_in,
+                                                                           const void *__restrict__ beta_in,
                                                                            CT *__restrict__ out)
 {
     using S = typename RT<DT>::S;
+    using PS = typename RT<PDT>::S;
+    const PS *gamma = (const PS *)gamma_in, *beta = (const PS *)beta_in;
     __shared__ CT lds[RowShape<WPR>::BW];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WPR;
@@ -976,12 +996,12 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_layernorm(const 
         const int i = chunk_start<VEC, WPR>(c, wr, lane);
         if (full || n >= VEC) {
             const int at = full ? i : chunk_at<VEC, WPR>(c, wr, lane, n);
-            if (gamma) load_vec16<CT, VEC>(gamma + at, g[c]);
-            if (beta) load_vec16<CT, VEC>(beta + at, b[c]);
+            if (gamma) load_params<PDT, VEC>(gamma + at, g[c]);
+            if (beta) load_params<PDT, VEC>(beta + at, b[c]);
         } else {
             for (int k = 0; k < VEC; k++) {
-                g[c][k] = gamma && i + k < n ? gamma[i + k] : (CT)1;
-                b[c][k] = beta && i + k < n ? beta[i + k] : (CT)0;
+                g[c][k] = gamma && i + k < n ? (CT)RT<PDT>::cv(gamma[i + k]) : (CT)1;
+                b[c][k] = beta && i + k < n ? (CT)RT<PDT>::cv(beta[i + k]) : (CT)0;
             }
         }
     }
@@ -1132,13 +1152,15 @@ __global__ __launch_bounds__(256) void k_row_softmax_stream(const void *__restri
     for (int i = threadIdx.x; i < n; i += blockDim.x) y[i] = (OS)(exp_c(RT<DT>::cv(x[i]) - m) / s);
 }
 
-template <int DT, typename CT>
+template <int DT, typename CT, int PDT>
 __global__ __launch_bounds__(256) void k_row_layernorm_stream(const void *__restrict__ xin, int n,
-                                                              CT eps, const CT *__restrict__ gamma,
-                                                              const CT *__restrict__ beta,
+                                                              CT eps, const void *__restrict__ gamma_in,
+                                                              const void *__restrict__ beta_in,
                                                               CT *__restrict__ out)
 {
     using S = typename RT<DT>::S;
+    using PS = typename RT<PDT>::S;
+    const PS *gamma = (const PS *)gamma_in, *beta = (const PS *)beta_in;
     __shared__ CT lds[4];
     const S *x = (const S *)xin + (size_t)blockIdx.x * (size_t)n;
     CT *y = out + (size_t)blockIdx.x * (size_t)n;
@@ -1153,8 +1175,8 @@ __global__ __launch_bounds__(256) void k_row_layernorm_stream(const void *__rest
     const CT dev = sqrt_c(block_allreduce_sum(q, lds) / (CT)n + eps);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         CT t = ((CT)RT<DT>::cv(x[i]) - mean) / dev;
-        if (gamma) t = t * gamma[i];
-        if (beta) t = t + beta[i];
+        if (gamma) t = t * (CT)RT<PDT>::cv(gamma[i]);
+        if (beta) t = t + (CT)RT<PDT>::cv(beta[i]);
         y[i] = t;
     }
 }
@@ -1623,7 +1645,7 @@ __device__ __forceinline__ void fold_store(void *out, int out_dt, size_t i, type
 // 153 us each on the generic kernels (a 120-byte state of every dtype, one
 // element per lane and load); sum, max, argmax and variance of it one after
 // another went from 359 to 124 us.
-template <int DT, int OP, int V>
+template <int DT, int OP, int V, bool NT>
 __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ xin, size_t n, size_t inner,
                                                       size_t slice, void *__restrict__ out, int out_dt,
                                                       int correction, int take_sqrt,
@@ -1655,7 +1677,7 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
             C v[4][V];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                if constexpr (V > 1) load_chunk<DT, V>(x + (r + 4 * u) * inner, v[u]);
+                if constexpr (V > 1) load_chunk<DT, V, NT>(x + (r + 4 * u) * inner, v[u]);
                 else v[u][0] = RT<DT>::cv(x[(r + 4 * u) * inner]);
             }
 #pragma unroll
@@ -1665,7 +1687,7 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
         }
         for (; r < hi; r += 4) {
             C v[V];
-            if constexpr (V > 1) load_chunk<DT, V>(x + r * inner, v);
+            if constexpr (V > 1) load_chunk<DT, V, NT>(x + r * inner, v);
             else v[0] = RT<DT>::cv(x[r * inner]);
 #pragma unroll
             for (int k = 0; k < V; k++) acc[k].add(v[k], (int)r);
@@ -2092,22 +2114,28 @@ static int result_dtype(int dtype, int rop)
     return dtype;
 }
 
-// Column launcher of k_col_reduce_t.  Columns are read in 16-byte packs
-// unless a row holds less than half a block of them (below that the lanes
-// left idle cost more than the narrower loads).  When the column blocks
-// cannot fill the GPU the rows are split into slices (at least 64 rows each,
-// at most 128 slices) merged by k_col_final_t; the number of slices counts
-// unaligned columns one by one, so the scratch they take stays within the
-// no-allocation entry's megabyte for the same calls.
+// Column launcher of k_col_reduce_t.  Columns are read in 16-byte packs,
+// nontemporally where the rows keep them aligned (chunks that cross lines
+// are cached: a line must outlive its first reader), unless a row holds less
+// than half a block of them.  When the column blocks cannot fill the GPU the
+// rows are split into slices (at least 64 rows each, at most 128 slices)
+// merged by k_col_final_t.  Sums of unaligned columns keep the number of
+// slices that 64-column blocks ask for, and so their order of additions and
+// a scratch that the no-allocation entry's megabyte holds for the same
+// calls; where 16-byte packs then leave fewer than two blocks a CU they are
+// read in narrower ones.  sum, max, argMax and var of [8000, 3001] bf16
+// along axis 0: 138 us with nontemporal loads and 264 blocks a call, 100 us.
 template <int DT, int OP>
 static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inner, void *out, int out_dt,
                                int correction, int take_sqrt, hipStream_t s)
 {
     using P = typename Fold<typename RT<DT>::C, OP>::P;
-    constexpr int V = RT<DT>::V;
+    constexpr int V = RT<DT>::V, W = sizeof(typename RT<DT>::S) == 2 ? 2 : 1;
+    constexpr bool ORDERED = OP == R_SUM || OP == R_MEAN || OP == R_PROD;
     const bool packed = inner % V == 0 && aligned16(x);
+    const size_t vec_blocks = (inner + 64 * V - 1) / (64 * V);
     const bool vec = packed || inner >= 32 * V;
-    const size_t split_blocks = (inner + (packed ? 64 * V : 64) - 1) / (packed ? 64 * V : 64);
+    const size_t split_blocks = packed || (vec && !ORDERED) ? vec_blocks : (inner + 63) / 64;
     size_t splits = 1;
     if (split_blocks * outer < 1024) {
         splits = (2048 + split_blocks * outer - 1) / (split_blocks * outer);
@@ -2120,12 +2148,17 @@ static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inn
     splits = (n + slice - 1) / slice;
     P *partial = nullptr;
     if (splits > 1) PT_TRY(scratch_alloc((void **)&partial, sizeof(P) * outer * splits * inner, s));
-    const size_t cols_per_block = vec ? 64 * V : 64;
-    dim3 grid((unsigned)((inner + cols_per_block - 1) / cols_per_block), (unsigned)splits, (unsigned)outer);
-    if (vec)
-        k_col_reduce_t<DT, OP, V><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, correction, take_sqrt, partial);
-    else
-        k_col_reduce_t<DT, OP, 1><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, correction, take_sqrt, partial);
+    const int width = !vec ? 1 : packed || !ORDERED || vec_blocks * splits * outer >= 512 ? V : W;
+    auto go = [&](auto N, auto T) {
+        constexpr int C = decltype(N)::value;
+        const dim3 grid((unsigned)((inner + 64 * C - 1) / (64 * C)), (unsigned)splits, (unsigned)outer);
+        k_col_reduce_t<DT, OP, C, decltype(T)::value><<<grid, 256, 0, s>>>(x, n, inner, slice, out, out_dt, correction,
+                                                                         take_sqrt, partial);
+    };
+    if (width == V && packed) go(std::integral_constant<int, V>{}, std::true_type{});
+    else if (width == V) go(std::integral_constant<int, V>{}, std::false_type{});
+    else if (W > 1 && width == W) go(std::integral_constant<int, W>{}, std::false_type{});
+    else go(std::integral_constant<int, 1>{}, std::false_type{});
     hipError_t e1 = hipGetLastError(), e2 = hipSuccess;
     if (splits > 1) {
         k_col_final_t<DT, OP><<<dim3((unsigned)((inner + 63) / 64), (unsigned)outer), 256, 0, s>>>(
@@ -2400,13 +2433,13 @@ static unsigned walk_grid(size_t rows)
     return (unsigned)(rows < b ? rows : b);
 }
 
-template <int DT, int NCH, int WPR, typename CT>
-static void launch_layernorm_nch(const void *x, size_t rows, int n, CT eps, const CT *g, const CT *b, CT *y,
+template <int DT, int NCH, int WPR, int PDT, typename CT>
+static void launch_layernorm_nch(const void *x, size_t rows, int n, CT eps, const void *g, const void *b, CT *y,
                                  hipStream_t s)
 {
     constexpr int V = RT<DT>::V, T = 64 * RowShape<WPR>::BW;
     auto go = [&](auto F) {
-        constexpr auto k = k_row_layernorm<DT, V, NCH, WPR, CT, decltype(F)::value>;
+        constexpr auto k = k_row_layernorm<DT, V, NCH, WPR, CT, PDT, decltype(F)::value>;
         // block-per-row kernels walk the rows (walk_grid blocks)
         unsigned grid;
         if constexpr (WPR == 1) grid = (unsigned)((rows + 3) / 4);
@@ -2417,32 +2450,32 @@ static void launch_layernorm_nch(const void *x, size_t rows, int n, CT eps, cons
     else go(std::false_type{});
 }
 
-template <int DT, typename CT>
-static void launch_layernorm_rows(const void *x, size_t rows, int n, CT eps, const CT *g,
-                                  const CT *b, CT *y, hipStream_t s)
+template <int DT, int PDT, typename CT>
+static void launch_layernorm_rows(const void *x, size_t rows, int n, CT eps, const void *g,
+                                  const void *b, CT *y, hipStream_t s)
 {
     constexpr int V = RT<DT>::V;
     const int chunks = (int)(((long long)n + 64 * V - 1) / (64 * V));
     if constexpr (DT == PT_FLOAT32 && sizeof(CT) == 4) {
         if (chunks > 4 && chunks <= 16 && row_waves() == 8)
-            return launch_layernorm_nch<DT, 2, 8>(x, rows, n, eps, g, b, y, s);
+            return launch_layernorm_nch<DT, 2, 8, PDT>(x, rows, n, eps, g, b, y, s);
     }
     switch (chunks) {
-    case 1: return launch_layernorm_nch<DT, 1, 1>(x, rows, n, eps, g, b, y, s);
-    case 2: return launch_layernorm_nch<DT, 2, 1>(x, rows, n, eps, g, b, y, s);
-    case 3: case 4: return launch_layernorm_nch<DT, 4, 1>(x, rows, n, eps, g, b, y, s);
+    case 1: return launch_layernorm_nch<DT, 1, 1, PDT>(x, rows, n, eps, g, b, y, s);
+    case 2: return launch_layernorm_nch<DT, 2, 1, PDT>(x, rows, n, eps, g, b, y, s);
+    case 3: case 4: return launch_layernorm_nch<DT, 4, 1, PDT>(x, rows, n, eps, g, b, y, s);
     default:
-        if (chunks <= 8) return launch_layernorm_nch<DT, 2, 4>(x, rows, n, eps, g, b, y, s);
-        if (chunks <= 16) return launch_layernorm_nch<DT, 4, 4>(x, rows, n, eps, g, b, y, s);
+        if (chunks <= 8) return launch_layernorm_nch<DT, 2, 4, PDT>(x, rows, n, eps, g, b, y, s);
+        if (chunks <= 16) return launch_layernorm_nch<DT, 4, 4, PDT>(x, rows, n, eps, g, b, y, s);
         // (gamma and beta stay in registers too: 8 chunks per lane at most)
-        if (chunks <= 32) return launch_layernorm_nch<DT, 8, 4>(x, rows, n, eps, g, b, y, s);
+        if (chunks <= 32) return launch_layernorm_nch<DT, 8, 4, PDT>(x, rows, n, eps, g, b, y, s);
         if constexpr (sizeof(CT) == 4) {
             // [3000, 13001] fp32: 83-98 us against 197 us for the streaming kernel
-            if (chunks <= 64) return launch_layernorm_nch<DT, 8, 8>(x, rows, n, eps, g, b, y, s);
+            if (chunks <= 64) return launch_layernorm_nch<DT, 8, 8, PDT>(x, rows, n, eps, g, b, y, s);
         }
         break;
     }
-    k_row_layernorm_stream<DT, CT><<<(unsigned)rows, 256, 0, s>>>(x, n, eps, g, b, y);
+    k_row_layernorm_stream<DT, CT, PDT><<<(unsigned)rows, 256, 0, s>>>(x, n, eps, g, b, y);
 }
 
 // Strided -> contiguous permuted copy used to move the softmax axis last.
@@ -2633,6 +2666,14 @@ pt_status pt_layernorm(const void *input, void *output, int input_dtype, int com
                        size_t rows, size_t n, double eps,
                        const void *gamma, const void *beta, pt_stream_t stream)
 {
+    return pt_layernorm_params(input, output, input_dtype, compute_dtype, rows, n, eps, gamma, beta, compute_dtype,
+                               stream);
+}
+
+pt_status pt_layernorm_params(const void *input, void *output, int input_dtype, int compute_dtype,
+                              size_t rows, size_t n, double eps,
+                              const void *gamma, const void *beta, int param_dtype, pt_stream_t stream)
+{
     PT_TRY(ensure_init());
     if (!(eps > 0.0) || !isfinite(eps))
         return fail(PT_ERR_INVALID, "LayerNorm epsilon must be finite and greater than zero");
@@ -2640,27 +2681,36 @@ pt_status pt_layernorm(const void *input, void *output, int input_dtype, int com
         return fail(PT_ERR_INVALID, "LayerNorm compute dtype must be float32 or float64");
     if (compute_dtype == PT_FLOAT32 && (!isfinite((float)eps) || (float)eps <= 0.0f))
         return fail(PT_ERR_INVALID, "LayerNorm epsilon is not representable as float32");
+    const bool half = input_dtype == PT_BFLOAT16 || input_dtype == PT_FLOAT16;
+    if (param_dtype != compute_dtype && !(compute_dtype == PT_FLOAT32 && half && param_dtype == input_dtype))
+        return fail(PT_ERR_INVALID, "LayerNorm parameters must have the compute dtype or a 16-bit input's");
     if (n == 0 && rows) return fail(PT_ERR_INVALID, "LayerNorm cannot normalize an empty dimension");
     if (n > (size_t)INT32_MAX) return fail(PT_ERR_INVALID, "LayerNorm row too long");
     if (!rows) return PT_OK;
     hipStream_t s = stream_of(stream);
-    int ni = (int)n;
+    const int ni = (int)n;
+    const void *g = gamma, *b = beta;
     if (compute_dtype == PT_FLOAT32) {
-        float e = (float)eps;
-        const float *g = (const float *)gamma, *b = (const float *)beta;
+        const float e = (float)eps;
         float *y = (float *)output;
+        auto go = [&](auto D, auto P) {
+            launch_layernorm_rows<decltype(D)::value, decltype(P)::value>(input, rows, ni, e, g, b, y, s);
+        };
+        using F = std::integral_constant<int, PT_FLOAT32>;
+        using B = std::integral_constant<int, PT_BFLOAT16>;
+        using H = std::integral_constant<int, PT_FLOAT16>;
+        const bool same = param_dtype == input_dtype;
         switch (input_dtype) {
-        case PT_FLOAT32: launch_layernorm_rows<PT_FLOAT32, float>(input, rows, ni, e, g, b, y, s); break;
-        case PT_BFLOAT16: launch_layernorm_rows<PT_BFLOAT16, float>(input, rows, ni, e, g, b, y, s); break;
-        case PT_FLOAT16: launch_layernorm_rows<PT_FLOAT16, float>(input, rows, ni, e, g, b, y, s); break;
+        case PT_FLOAT32: go(F{}, F{}); break;
+        case PT_BFLOAT16: same ? go(B{}, B{}) : go(B{}, F{}); break;
+        case PT_FLOAT16: same ? go(H{}, H{}) : go(H{}, F{}); break;
         default: return fail(PT_ERR_INVALID, "float32 layerNorm takes f32/f16/bf16 input");
         }
     } else {
-        const double *g = (const double *)gamma, *b = (const double *)beta;
         double *y = (double *)output;
         switch (input_dtype) {
-        case PT_FLOAT64: launch_layernorm_rows<PT_FLOAT64, double>(input, rows, ni, eps, g, b, y, s); break;
-        case PT_FLOAT32: launch_layernorm_rows<PT_FLOAT32, double>(input, rows, ni, eps, g, b, y, s); break;
+        case PT_FLOAT64: launch_layernorm_rows<PT_FLOAT64, PT_FLOAT64>(input, rows, ni, eps, g, b, y, s); break;
+        case PT_FLOAT32: launch_layernorm_rows<PT_FLOAT32, PT_FLOAT64>(input, rows, ni, eps, g, b, y, s); break;
         default: return fail(PT_ERR_INVALID, "float64 layerNorm takes f64/f32 input");
         }
     }

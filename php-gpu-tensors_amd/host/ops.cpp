@@ -567,14 +567,18 @@ TensorP cuda_array_layernorm(const TensorP &a, const int *axes_in, int naxes, do
     for (int i = 0; i < naxes; i++) n *= (size_t)a->shape[sorted[i]];
     size_t rows = n ? a->numel() / n : 0;
 
-    // parameters: dims follow `axes`; reorder them to ascending-axis order
+    // parameters: dims follow `axes`; reorder them to ascending-axis order.
+    // Parameters of a 16-bit input's own dtype are widened by the kernel.
+    auto as_input = [&](const TensorP &p) { return !p || p->dtype == xp->dtype; };
+    const bool half = xp->dtype == PT_BFLOAT16 || xp->dtype == PT_FLOAT16;
+    const int pdt = cdt == PT_FLOAT32 && half && (scale || bias) && as_input(scale) && as_input(bias) ? xp->dtype : cdt;
     auto prep = [&](const TensorP &p) -> TensorP {
         if (!p) return nullptr;
         int pperm[kMaxDims];
         for (int i = 0; i < naxes; i++)
             for (int j = 0; j < naxes; j++)
                 if (axes[j] == sorted[i]) pperm[i] = j;
-        TensorP q = tensor_cast(p, cdt);
+        TensorP q = tensor_cast(p, pdt);
         if (!q) return nullptr;
         q = transpose(q, pperm, naxes);
         if (!q) return nullptr;
@@ -587,8 +591,8 @@ TensorP cuda_array_layernorm(const TensorP &a, const int *axes_in, int naxes, do
     for (int d = 0; d < a->ndims; d++) pshape[d] = a->shape[perm[d]];
     TensorP outp = identity ? output_tensor(pshape, a->ndims, cdt) : make_empty(pshape, a->ndims, cdt);
     if (!outp) return nullptr;
-    if (rows && !check_status(pt_layernorm(xp->data(), outp->storage->ptr, xp->dtype, cdt, rows, n, eps,
-                                           g ? g->data() : nullptr, b ? b->data() : nullptr, nullptr),
+    if (rows && !check_status(pt_layernorm_params(xp->data(), outp->storage->ptr, xp->dtype, cdt, rows, n, eps,
+                                                  g ? g->data() : nullptr, b ? b->data() : nullptr, pdt, nullptr),
                               "LayerNorm kernel failed"))
         return nullptr;
     if (identity) return outp;

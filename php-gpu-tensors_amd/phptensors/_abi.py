@@ -112,6 +112,8 @@ SIGNATURES = {
                                   ctypes.c_int, ctypes.c_int, vp]),
     "pt_layernorm": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_size_t,
                                     ctypes.c_size_t, ctypes.c_double, vp, vp, vp]),
+    "pt_layernorm_params": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_size_t,
+                                           ctypes.c_size_t, ctypes.c_double, vp, vp, ctypes.c_int, vp]),
     "pt_matmul": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, c_int_p, c_size_p, ctypes.c_int,
                                  c_int_p, c_size_p, ctypes.c_int, c_int_p, ctypes.c_int, vp]),
     "pt_matmul_tune": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, c_int_p, c_size_p, ctypes.c_int,

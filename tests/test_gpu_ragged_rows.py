@@ -89,3 +89,20 @@ def test_ragged_nonfinite_rows():
         soft = a.softmax(1).toNumpy()
         assert np.all(np.isnan(soft[[0, 1, 3, 4]][:, 0])) and np.all(np.isfinite(soft[[2, 5]]))
         assert soft[2, n - 1] == 0.0
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("n", [1, 7, 8, 512, 1001, 4096, 16385, 40000])
+def test_layernorm_parameters_of_the_inputs_type(dt, n):
+    """Scale and bias in the input's 16-bit type give the bits that their
+    widened values give, together or alone; mixed types still cast."""
+    from phptensors import CudaArray, synthetic
+    code = {"bfloat16": O.BF16, "float16": O.F16}[dt]
+    up = lambda v: CudaArray.fromNumpy(O.to_storage(v, code), dt)  # noqa: E731
+    x = up(synthetic.normal((4, n), 0.5, 2.0, seed=n))
+    g, b = up(synthetic.normal((n,), 1.0, 0.2, seed=1)), up(synthetic.normal((n,), 0.0, 0.2, seed=2))
+    gf, bf = g.astype("float32"), b.astype("float32")
+    bits = lambda s, t: x.layerNorm([1], 1e-5, s, t).toBits().view(np.uint32)  # noqa: E731
+    ref = bits(gf, bf)
+    assert np.array_equal(bits(g, b), ref) and np.array_equal(bits(g, bf), ref)
+    assert np.array_equal(bits(g, None), bits(gf, None)) and np.array_equal(bits(None, b), bits(None, bf))
