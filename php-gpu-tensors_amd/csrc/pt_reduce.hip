@@ -2120,11 +2120,12 @@ static int result_dtype(int dtype, int rop)
 // than half a block of them.  When the column blocks cannot fill the GPU the
 // rows are split into slices (at least 64 rows each, at most 128 slices)
 // merged by k_col_final_t.  Sums of unaligned columns keep the number of
-// slices that 64-column blocks ask for, and so their order of additions and
-// a scratch that the no-allocation entry's megabyte holds for the same
-// calls; where 16-byte packs then leave fewer than two blocks a CU they are
+// slices that 64-column blocks ask for, and so their order of additions;
+// maxima and minima take more only while their scratch stays within the
+// no-allocation entry's megabyte, which then holds it for the same calls as
+// ever.  Where 16-byte packs leave sums fewer than two blocks a CU they are
 // read in narrower ones.  sum, max, argMax and var of [8000, 3001] bf16
-// along axis 0: 138 us with nontemporal loads and 264 blocks a call, 100 us.
+// along axis 0: 138 us with nontemporal loads and 264 blocks a call, 102 us.
 template <int DT, int OP>
 static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inner, void *out, int out_dt,
                                int correction, int take_sqrt, hipStream_t s)
@@ -2135,14 +2136,21 @@ static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inn
     const bool packed = inner % V == 0 && aligned16(x);
     const size_t vec_blocks = (inner + 64 * V - 1) / (64 * V);
     const bool vec = packed || inner >= 32 * V;
-    const size_t split_blocks = packed || (vec && !ORDERED) ? vec_blocks : (inner + 63) / 64;
-    size_t splits = 1;
-    if (split_blocks * outer < 1024) {
-        splits = (2048 + split_blocks * outer - 1) / (split_blocks * outer);
-        size_t max_splits = n / 64;
-        if (splits > max_splits) splits = max_splits;
-        if (splits > 128) splits = 128;
-        if (splits < 1) splits = 1;
+    auto slices_for = [&](size_t col_blocks) -> size_t {
+        const size_t blocks = col_blocks * outer;
+        if (blocks >= 1024) return 1;
+        const size_t most = n / 64 < 128 ? n / 64 : 128, want = (2048 + blocks - 1) / blocks;
+        const size_t k = want < most ? want : most;
+        return k > 1 ? k : 1;
+    };
+    size_t splits = slices_for(packed ? vec_blocks : (inner + 63) / 64);
+    if (!packed && vec && !ORDERED) {
+        size_t more = slices_for(vec_blocks);
+        if constexpr (OP == R_MAX || OP == R_MIN) {
+            const size_t held = ((size_t)PT_STATIC_SCRATCH_BYTES) / (sizeof(P) * outer * inner);
+            if (more > held) more = held;
+        }
+        if (more > splits) splits = more;
     }
     const size_t slice = (n + splits - 1) / splits;
     splits = (n + slice - 1) / slice;

@@ -110,3 +110,23 @@ def test_global_reduction_of_an_offset_view(G):
         v = CudaArray.fromNumpy(xs, "bfloat16").slice([off, None])
         assert v.sum().item() == float(x[off:].sum())
         assert v.argMax().item() == int(np.argmax(x[off:]))
+
+
+@pytest.mark.parametrize("shape", [(1000, 18075), (8000, 3001), (700, 66001)], ids=str)
+@pytest.mark.parametrize("op", ["max", "min", "sum"])
+def test_unaligned_columns_fit_the_static_scratch(shape, op):
+    """Column reductions whose slices of 64-column blocks fit the megabyte of
+    the no-allocation entry still fit it, with pt_reduce's bits."""
+    from phptensors import _abi as A
+    x = np.random.default_rng(4).integers(0, 0x3F80, shape, dtype=np.uint16)
+    rows, cols = shape
+    dx, one, two = A.to_device(x), A.DeviceBuffer(cols * 4), A.DeviceBuffer(cols * 4)
+    lib = A.load()
+    args = (A.BFLOAT16, A.OP[op], A.ints(shape), A.sizes([cols, 1]), 2, 0, 0, None)
+    A.check(lib.pt_reduce_noalloc(dx.ptr, one.ptr, *args), "reduction without allocation")
+    A.check(lib.pt_reduce(dx.ptr, two.ptr, *args), "reduction")
+    got = one.download(np.float32, (cols,))
+    assert np.array_equal(got, two.download(np.float32, (cols,)))
+    if op != "sum":
+        ref = O.from_storage(x, O.BF16).astype(np.float32)
+        assert np.array_equal(got, ref.max(0) if op == "max" else ref.min(0))
