@@ -169,6 +169,80 @@ struct RowDiv {
 __device__ __forceinline__ float sqrt_c(float a) { return sqrtf(a); }
 __device__ __forceinline__ double sqrt_c(double a) { return sqrt(a); }
 
+// v of the lane that DPP control CTRL names, added.
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+    return v + __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
+}
+
+// Sums over the wave of two doubles at once: s in lanes 0..31, q in lanes
+// 32..63 (the first exchange gives each half-wave its own sum to finish, so
+// that the two cost the steps of one).
+__device__ __forceinline__ double wave_sums(double s, double q)
+{
+    const unsigned long long sb = __builtin_bit_cast(unsigned long long, s);
+    const unsigned long long qb = __builtin_bit_cast(unsigned long long, q);
+    auto join = [](unsigned lo, unsigned hi) {
+        return __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
+    };
+    auto lo = __builtin_amdgcn_permlane32_swap((unsigned)sb, (unsigned)qb, false, false);
+    auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(sb >> 32), (unsigned)(qb >> 32), false, false);
+    double v = join(lo[0], hi[0]) + join(lo[1], hi[1]);
+    const unsigned long long vb = __builtin_bit_cast(unsigned long long, v);
+    lo = __builtin_amdgcn_permlane16_swap((unsigned)vb, (unsigned)vb, false, false);
+    hi = __builtin_amdgcn_permlane16_swap((unsigned)(vb >> 32), (unsigned)(vb >> 32), false, false);
+    v = join(lo[0], hi[0]) + join(lo[1], hi[1]);
+    v = add_dpp<0x140>(v);     // row_mirror
+    v = add_dpp<0x141>(v);     // row_half_mirror
+    v = add_dpp<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+    return add_dpp<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+}
+
+// Variance state of a row of 32- or 16-bit floats: the sum of the elements'
+// deviations from the row's first element and the sum of their squares, in
+// double.  No sum can leave double's range, a row of one value gives 0, and
+// (first - mean)^2 <= n x variance, so the subtraction at the end loses at
+// most a factor n of 2^-53.  An infinite or NaN element makes the result NaN
+// (inf - inf).
+struct DevSum {
+    double s, q;
+    __device__ void add(double d)
+    {
+        s = s + d;
+        q = __builtin_fma(d, d, q);
+    }
+};
+
+// The row's variance from its lanes' sums (in lane 0 of its first wave);
+// rn = 1 / n, rc = 1 / (n - correction).  Every wave of a WPR > 1 block comes
+// here.
+template <int WPR>
+__device__ __forceinline__ double dev_variance(const DevSum &d, double rn, double rc)
+{
+    double v = wave_sums(d.s, d.q);
+    if constexpr (WPR > 1) {
+        __shared__ double part[2][WPR];
+        const int lane = threadIdx.x & 63, half = lane >> 5, l = lane & 31;
+        if (l == 0) part[half][threadIdx.x >> 6] = v;
+        __syncthreads();
+        if (threadIdx.x >= 64) return 0.0;
+        v = part[half][l & (WPR - 1)];
+        v = add_dpp<0xB1>(v);
+        v = add_dpp<0x4E>(v);
+        if constexpr (WPR == 8) v = add_dpp<0x141>(v);
+    }
+    const unsigned long long vb = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)vb, 32);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(vb >> 32), 32);
+    const double q = __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
+    const double m2 = q - v * (v * rn);
+    return (m2 < 0.0 ? 0.0 : m2) * rc;
+}
+
 // Moments state for var/std (Chan et al. parallel combination of Welford
 // states, reduction_ops.cuh:97-112).
 struct Mom {
@@ -250,7 +324,6 @@ template <typename C, bool MAXIMIZE> struct ArgAcc {
 template <typename C> struct Acc<C, R_ARGMAX> : ArgAcc<C, true> {};
 template <typename C> struct Acc<C, R_ARGMIN> : ArgAcc<C, false> {};
 template <typename C> struct Acc<C, R_VAR> {
-    Mom m = {0, 0, 0};
     C cn = 0, cmean = 0, cm2 = 0;  // running per-lane state in compute type
     __device__ void add(C v, int)
     {
@@ -263,6 +336,11 @@ template <typename C> struct Acc<C, R_VAR> {
         cn = n1;
     }
     __device__ Mom lane_state() const { return Mom{(double)cn, (double)cmean, (double)cm2}; }
+};
+template <> struct Acc<float, R_VAR> {
+    double first = 0;  // of the row
+    DevSum d = {0, 0};
+    __device__ void add(float v, int) { d.add((double)v - first); }
 };
 
 template <typename C, int OP>
@@ -306,16 +384,21 @@ __device__ __forceinline__ void wave_merge(Acc<C, OP> &a)
     }
 }
 
-// Chunk-level variance update: V elements at once (exact two-pass on the
-// registers of the chunk, then a Chan combine), one division per chunk.
+// Chunk-level variance update: V elements at once.  float64: exact two-pass
+// on the registers of the chunk, then a Chan combine, one division per chunk
+// (the elements are scaled by 1 / V, a power of two, before they are added,
+// so that the chunk's sum stays in range).
 template <typename C, int V>
 __device__ __forceinline__ void var_add_chunk(Acc<C, R_VAR> &a, const C (&v)[V], int valid)
 {
-    if (valid == V) {
-        C s = 0;
+    if constexpr (sizeof(C) == 4) {
 #pragma unroll
-        for (int k = 0; k < V; k++) s = s + v[k];
-        C mb = s / (C)V;
+        for (int k = 0; k < V; k++)
+            if (k < valid) a.add(v[k], 0);
+    } else if (valid == V) {
+        C mb = 0;
+#pragma unroll
+        for (int k = 0; k < V; k++) mb = mb + v[k] * ((C)1 / (C)V);
         C m2b = 0;
 #pragma unroll
         for (int k = 0; k < V; k++) {
@@ -382,7 +465,8 @@ __device__ __forceinline__ int row_head(const S *x, int n)
 template <int DT, int OP, int VEC, int WPR, bool RAG = false>
 __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_reduce(const void *__restrict__ xin, size_t rows,
                                                                         int n, size_t ld, void *__restrict__ out,
-                                                                        int out_dt, int correction, int take_sqrt)
+                                                                        int out_dt, int correction, int take_sqrt,
+                                                                        double rn, double rc)
 {
     using S = typename RT<DT>::S;
     using C = typename RT<DT>::C;
@@ -396,6 +480,8 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_reduce(const voi
     if (row >= rows) return;                          // uniform per block when WPR > 1
     const S *x = (const S *)xin + row * ld;
     Acc<C, OP> acc;
+    constexpr bool DEV = OP == R_VAR && sizeof(C) == 4;
+    if constexpr (DEV) acc.first = (double)RT<DT>::cv(x[0]);
     constexpr int STEP = 64 * VEC;                    // one wave-wide chunk
     constexpr int RSTEP = WPR * STEP;                 // one row-wide chunk
     if constexpr (RAG) {
@@ -483,7 +569,10 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_reduce(const voi
             }
         }
     }
-    if constexpr (OP == R_VAR) {
+    if constexpr (DEV) {
+        const double var = dev_variance<WPR>(acc.d, rn, rc);
+        if (wr == 0 && lane == 0) store_out(out, out_dt, row, take_sqrt ? sqrt(var) : var);
+    } else if constexpr (OP == R_VAR) {
         Mom m = acc.lane_state();
 #pragma unroll
         for (int s = 32; s >= 1; s >>= 1) m = mom_combine(m, mom_shfl(m, s));
@@ -699,48 +788,69 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_arg2(const void 
     ((int32_t *)out)[row] = m == ident ? 0 : idx;
 }
 
-// Variance / standard deviation: exact two-pass form (mean, then the sum of
-// squared deviations from it) over the values held in registers.  Same
-// result definition as the Welford kernels (M2 / (n - correction), sqrt for
-// std), one HBM pass.
+// Variance / standard deviation of rows held in registers, one HBM pass.
+// 32- and 16-bit rows: DevSum, one exchange between the waves ([8192, 4096]
+// fp32 18.7 us, [100000, 100] 19.7 us; float32 means and deviations, whose
+// sums and squares left the type's range, took 19.8 and 21.9).  float64 rows:
+// exact two-pass form (mean, as the row's first element plus the mean of the
+// deviations from it, then the sum of squared deviations from the mean).
+// Same result definition as the Welford kernels (M2 / (n - correction), sqrt
+// for std).
 template <int DT, int VEC, int NCH, int WPR, bool RAG = false>
 __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_moments(const void *__restrict__ xin, size_t rows,
                                                                          int n, size_t ld, void *__restrict__ out,
-                                                                         int out_dt, int correction, int take_sqrt)
+                                                                         int out_dt, int correction, int take_sqrt,
+                                                                         double rn, double rc)
 {
     using S = typename RT<DT>::S;
     using C = typename RT<DT>::C;
-    __shared__ C lds[RowShape<WPR>::BW];
+    constexpr int BW = RowShape<WPR>::BW;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WPR;
     const size_t row = (size_t)blockIdx.x * RowShape<WPR>::RPB + wave / WPR;
     if (row >= rows) return;  // WPR > 1: one row per block, never taken
     const S *x = (const S *)xin + row * ld;
+    // elements that a lane does not own hold the row's first one: they
+    // deviate from it by 0
+    const C first = RT<DT>::cv(x[0]);
     C v[NCH][VEC];
     // (ragged rows: chunks from the first whole line, as k_row_reduce)
     int head = 0;
-    C vh = 0;
+    C vh = first;
     bool has_head = false;
     if constexpr (RAG) {
         head = row_head(x, n);
         has_head = wr == 0 && lane < head;
         if (has_head) vh = RT<DT>::cv(x[lane]);
     }
-    const bool full = load_row<DT, VEC, NCH, WPR, true, true>(x + head, n - head, wr, lane, (C)0, v);
+    const bool full = load_row<DT, VEC, NCH, WPR, true, true>(x + head, n - head, wr, lane, first, v);
+    if constexpr (sizeof(C) == 4) {
+        const double at = (double)first;
+        DevSum d = {0, 0};
+        if constexpr (RAG) d.add((double)vh - at);
+#pragma unroll
+        for (int c = 0; c < NCH; c++)
+#pragma unroll
+            for (int k = 0; k < VEC; k++) d.add((double)v[c][k] - at);
+        const double var = dev_variance<WPR>(d, rn, rc);
+        if (wr == 0 && lane == 0) store_out(out, out_dt, row, take_sqrt ? sqrt(var) : var);
+        return;
+    }
+    __shared__ C lds[BW];
     if (!RAG && n == NCH * VEC * 64 * WPR) {
         // Every lane holds NCH * VEC elements: exact two-pass over the
         // lane's own values, then Chan's pairwise combination of
         // (mean, M2) states of equal counts over the lanes (butterfly: both
         // partners compute the same sums, so every lane ends with the wave's
-        // state) and over the waves, in double, by one lane: one exchange
-        // through LDS instead of a row mean followed by a row sum.
+        // state) and over the waves, by one lane: one exchange through LDS
+        // instead of a row mean followed by a row sum.
         constexpr int NL = NCH * VEC;
         C ls = 0;
 #pragma unroll
         for (int c = 0; c < NCH; c++)
 #pragma unroll
-            for (int k = 0; k < VEC; k++) ls = ls + v[c][k];
-        C mean = ls / (C)NL, q = 0;
+            for (int k = 0; k < VEC; k++) ls = ls + (v[c][k] - first);
+        C mean = first + ls / (C)NL, q = 0;
 #pragma unroll
         for (int c = 0; c < NCH; c++)
 #pragma unroll
@@ -749,54 +859,26 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_moments(const vo
                 q = q + d * d;
             }
         C cnt = (C)NL;
-        // equal-count combination of the partner's state (om, oq)
-        auto chan = [&](C om, C oq) {
+#pragma unroll
+        for (int sh = 32; sh >= 1; sh >>= 1) {
+            // equal-count combination of the partner's state (om, oq)
+            const C om = __shfl_xor(mean, sh, PT_WAVE), oq = __shfl_xor(q, sh, PT_WAVE);
             const C d = om - mean;
             q = (q + oq) + d * d * (cnt * (C)0.5);
-            mean = (mean + om) * (C)0.5;
+            mean = mean * (C)0.5 + om * (C)0.5;
             cnt = cnt * 2;
-        };
-        if constexpr (sizeof(C) == 4) {
-            // lanes ^ 1, ^ 2 (DPP quad permutes), then the half-row and row
-            // mirrors (as in wave_all), then the four row states in order
-            auto dpp = [](C x, auto CTRL) {
-                return __builtin_bit_cast(C, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
-                                                                          decltype(CTRL)::value, 0xF, 0xF, false));
-            };
-            chan(dpp(mean, std::integral_constant<int, 0xB1>{}), dpp(q, std::integral_constant<int, 0xB1>{}));
-            chan(dpp(mean, std::integral_constant<int, 0x4E>{}), dpp(q, std::integral_constant<int, 0x4E>{}));
-            chan(dpp(mean, std::integral_constant<int, 0x141>{}), dpp(q, std::integral_constant<int, 0x141>{}));
-            chan(dpp(mean, std::integral_constant<int, 0x140>{}), dpp(q, std::integral_constant<int, 0x140>{}));
-            auto rl = [](C x, int l) {
-                return __builtin_bit_cast(C, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
-            };
-            const C m16 = rl(mean, 16), q16 = rl(q, 16), m32 = rl(mean, 32), q32 = rl(q, 32);
-            const C m48 = rl(mean, 48), q48 = rl(q, 48);
-            mean = rl(mean, 0);
-            q = rl(q, 0);
-            const C c16 = cnt;
-            chan(m16, q16);  // rows 0 + 1
-            const C ma = mean, qa = q;
-            mean = m32;
-            q = q32;
-            cnt = c16;
-            chan(m48, q48);  // rows 2 + 3
-            chan(ma, qa);    // (rows 2 + 3) + (rows 0 + 1): equal counts, symmetric
-        } else {
-#pragma unroll
-            for (int sh = 32; sh >= 1; sh >>= 1) chan(__shfl_xor(mean, sh, PT_WAVE), __shfl_xor(q, sh, PT_WAVE));
         }
         if constexpr (WPR > 1) {
-            __shared__ C part_m[RowShape<WPR>::BW], part_q[RowShape<WPR>::BW];
+            __shared__ C part_m[BW], part_q[BW];
             if (lane == 0) {
                 part_m[wave] = mean;
                 part_q[wave] = q;
             }
             __syncthreads();
             if (wr != 0 || lane != 0) return;
-            double dm = (double)mean, dq = (double)q, dn = (double)cnt;
+            double dm = mean, dq = q, dn = cnt;
             for (int w = 1; w < WPR; w++) {
-                const double om = (double)part_m[wave + w], oq = (double)part_q[wave + w], on = (double)cnt;
+                const double om = part_m[wave + w], oq = part_q[wave + w], on = cnt;
                 const double nn = dn + on, d = om - dm;
                 dm = dm + d * (on / nn);
                 dq = dq + oq + d * d * (dn * on / nn);
@@ -805,17 +887,17 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_moments(const vo
             const double var = dq / (double)(n - correction);
             store_out(out, out_dt, row, take_sqrt ? sqrt(var) : var);
         } else if (lane == 0) {
-            const double var = (double)q / (double)(n - correction);
+            const double var = q / (double)(n - correction);
             store_out(out, out_dt, row, take_sqrt ? sqrt(var) : var);
         }
         return;
     }
-    C s = vh;
+    C s = vh - first;
 #pragma unroll
     for (int c = 0; c < NCH; c++)
 #pragma unroll
-        for (int k = 0; k < VEC; k++) s = s + v[c][k];
-    const C mean = row_sum<C, WPR>(s, lds) / (C)n;
+        for (int k = 0; k < VEC; k++) s = s + (v[c][k] - first);
+    const C mean = first + row_sum<C, WPR>(s, lds) / (C)n;
     C q = 0;
     if (has_head) q = (vh - mean) * (vh - mean);
     // Infinities poison the result as in Welford without a per-element term:
@@ -842,7 +924,7 @@ __global__ __launch_bounds__(64 * RowShape<WPR>::BW) void k_row_moments(const vo
     }
     q = row_sum<C, WPR>(q, lds);
     if (wr == 0 && lane == 0) {
-        double var = (double)q / (double)(n - correction);
+        const double var = q / (double)(n - correction);
         store_out(out, out_dt, row, take_sqrt ? sqrt(var) : var);
     }
 }
@@ -1980,8 +2062,7 @@ static bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 // Waves per row of the block-per-row kernels on fp32 rows of 5 to 16
 // chunks of 16 bytes per wave-row step (up to 4096 floats): 8 for every op.
 // On config 2 (X[8192, 4096]) against 4 waves: sum 20.5 against 20.8 us,
-// softmax 41.6 against 42.9 us, layerNorm 43.4 against 43.9 us, variance
-// (single-exchange Chan merge) 20.9-21.0 against 21.1; argmax / argmin with
+// softmax 41.6 against 42.9 us, layerNorm 43.4 against 43.9 us; argmax / argmin with
 // the two-pass k_row_arg2 20.4-20.5 against 21.3-21.4 us for the 4-wave
 // (value, index) kernel (8 waves of that kernel took 22.8 us).  16 waves
 // (1024-thread blocks) ran 30-60 % slower for every op, and nontemporal row
@@ -2014,49 +2095,50 @@ static void launch_rows_wide(const void *x, size_t rows, int n, size_t ld, void 
     dim3 block(256);
     const int chunks = (int)(((long long)n + 64 * V - 1) / (64 * V));
     dim3 grid1((unsigned)rows), grid4((unsigned)((rows + 3) / 4));
+    const double rn = 1.0 / (double)n, rc = 1.0 / (double)(n - correction);
     if constexpr (DT == PT_FLOAT32) {
         if (row_waves() == 8 && chunks > 4 && chunks <= 16) {
             dim3 block8(512);
             if constexpr (OP == R_VAR)
                 k_row_moments<DT, V, 2, 8, RAG><<<grid1, block8, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                        take_sqrt);
+                                                                        take_sqrt, rn, rc);
             else if constexpr (OP == R_ARGMAX || OP == R_ARGMIN)
                 k_row_arg2<V, 2, 8, OP == R_ARGMAX, RAG><<<grid1, block8, 0, s>>>(x, rows, n, ld, out);
             else
-                k_row_reduce<DT, OP, V, 8, RAG><<<grid1, block8, 0, s>>>(x, rows, n, ld, out, out_dt, 0, 0);
+                k_row_reduce<DT, OP, V, 8, RAG><<<grid1, block8, 0, s>>>(x, rows, n, ld, out, out_dt, 0, 0, rn, rc);
             return;
         }
     }
     if constexpr (OP == R_VAR) {
-        // rows that fit in registers: two-pass moments, a wave per row up to
-        // 4 chunks a lane, a block per row beyond
+        // rows that fit in registers: a wave per row up to 4 chunks a lane, a
+        // block per row beyond
         if (chunks <= 32) {
             if (chunks == 1)
                 k_row_moments<DT, V, 1, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                        take_sqrt);
+                                                                        take_sqrt, rn, rc);
             else if (chunks == 2)
                 k_row_moments<DT, V, 2, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                        take_sqrt);
+                                                                        take_sqrt, rn, rc);
             else if (chunks <= 4)
                 k_row_moments<DT, V, 4, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                        take_sqrt);
+                                                                        take_sqrt, rn, rc);
             else if (chunks <= 8)
                 k_row_moments<DT, V, 2, 4, RAG><<<grid1, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                       take_sqrt);
+                                                                       take_sqrt, rn, rc);
             else if (chunks <= 16)
                 k_row_moments<DT, V, 4, 4, RAG><<<grid1, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                       take_sqrt);
+                                                                       take_sqrt, rn, rc);
             else
                 k_row_moments<DT, V, 8, 4, RAG><<<grid1, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction,
-                                                                       take_sqrt);
+                                                                       take_sqrt, rn, rc);
             return;
         }
     }
     // long rows: a block per row (16 chunks of 16 B in flight per row)
     if (n >= 4 * 64 * V * 2)
-        k_row_reduce<DT, OP, V, 4, RAG><<<grid1, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt);
+        k_row_reduce<DT, OP, V, 4, RAG><<<grid1, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt, rn, rc);
     else
-        k_row_reduce<DT, OP, V, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt);
+        k_row_reduce<DT, OP, V, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt, rn, rc);
 }
 
 template <int DT, int OP>
@@ -2070,7 +2152,7 @@ static void launch_rows_t(const void *x, size_t rows, int n, size_t ld, void *ou
         launch_rows_wide<DT, OP, true>(x, rows, n, ld, out, out_dt, correction, take_sqrt, s);
     else
         k_row_reduce<DT, OP, 1, 1><<<dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s>>>(
-            x, rows, n, ld, out, out_dt, correction, take_sqrt);
+            x, rows, n, ld, out, out_dt, correction, take_sqrt, 1.0 / (double)n, 1.0 / (double)(n - correction));
 }
 
 template <int DT>
