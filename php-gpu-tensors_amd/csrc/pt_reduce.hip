@@ -1672,12 +1672,13 @@ template <typename C, int OP> struct ArgFold {
 };
 template <typename C> struct Fold<C, R_ARGMAX> : ArgFold<C, R_ARGMAX> {};
 template <typename C> struct Fold<C, R_ARGMIN> : ArgFold<C, R_ARGMIN> {};
-// Moments in double, as sums of the deviations from the lane's first value
-// and of their squares: two additions and a multiplication an element where
-// Welford's step has a division.  The shift is one of the values, so the
-// subtraction at the end loses at most a factor of the lane's count
-// ((shift - mean)^2 <= count x variance), and an infinite or NaN element
-// still makes the result NaN (inf - inf).
+// Moments of 32- and 16-bit floats in double, as sums of the deviations from
+// the lane's first value and of their squares: two additions and a
+// multiplication an element where Welford's step has a division.  The shift
+// is one of the values, so the subtraction at the end loses at most a factor
+// of the lane's count of 2^-53 ((shift - mean)^2 <= count x variance), which
+// the rounding of the result to 32 bits covers, and an infinite or NaN
+// element still makes the result NaN (inf - inf).
 template <typename C> struct Fold<C, R_VAR> {
     using P = Mom;
     double shift = 0, s = 0, q = 0;
@@ -1697,6 +1698,37 @@ template <typename C> struct Fold<C, R_VAR> {
     __device__ static P none() { return Mom{0, 0, 0}; }
     __device__ static P merge(P x, P y) { return mom_combine(x, y); }
 };
+// Moments of float64: no wider type covers that loss, so Welford's updates,
+// four elements to a division where the kernel has four at hand.
+template <> struct Fold<double, R_VAR> {
+    using P = Mom;
+    Acc<double, R_VAR> a;
+    __device__ void begin(double) {}
+    __device__ void add(double v, int) { a.add(v, 0); }
+    __device__ void add4(double v0, double v1, double v2, double v3)
+    {
+        const double v[4] = {v0, v1, v2, v3};
+        var_add_chunk<double, 4>(a, v, 4);
+    }
+    __device__ P part(size_t) const { return a.lane_state(); }
+    __device__ static P none() { return Mom{0, 0, 0}; }
+    __device__ static P merge(P x, P y) { return mom_combine(x, y); }
+};
+
+// Four elements (rows or chunks i, i + step, ...) folded into each of V states.
+template <typename C, int OP, int V>
+__device__ __forceinline__ void fold4(Fold<C, OP> (&acc)[V], const C (&v)[4][V], size_t i, size_t step, int k_step)
+{
+    if constexpr (OP == R_VAR && sizeof(C) == 8) {
+#pragma unroll
+        for (int k = 0; k < V; k++) acc[k].add4(v[0][k], v[1][k], v[2][k], v[3][k]);
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int k = 0; k < V; k++) acc[k].add(v[u][k], (int)(i + u * step + k * k_step));
+    }
+}
 
 template <typename C, int OP>
 __device__ __forceinline__ void fold_store(void *out, int out_dt, size_t i, typename Fold<C, OP>::P p, size_t n,
@@ -1762,10 +1794,7 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
                 if constexpr (V > 1) load_chunk<DT, V, NT>(x + (r + 4 * u) * inner, v[u]);
                 else v[u][0] = RT<DT>::cv(x[(r + 4 * u) * inner]);
             }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int k = 0; k < V; k++) acc[k].add(v[u][k], (int)(r + 4 * u));
+            fold4<C, OP, V>(acc, v, r, 4, 0);
         }
         for (; r < hi; r += 4) {
             C v[V];
@@ -1781,6 +1810,11 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
 #pragma unroll
         for (int k = 0; k < V; k++)
             if (k < valid && r < hi) acc[k].begin(RT<DT>::cv(x[r * inner + k]));
+        if constexpr (OP == R_VAR && sizeof(C) == 8) {
+            static_assert(V <= 2, "one column is left of a float64 pack");
+            for (; r + 12 < hi; r += 16)
+                acc[0].add4(x[r * inner], x[(r + 4) * inner], x[(r + 8) * inner], x[(r + 12) * inner]);
+        }
         for (; r < hi; r += 4)
 #pragma unroll
             for (int k = 0; k < V; k++)
@@ -1917,10 +1951,7 @@ __global__ __launch_bounds__(256) void k_glob_reduce_t(
         C v[U][V];
 #pragma unroll
         for (int u = 0; u < U; u++) load_chunk<DT, V>(x + i + u * step, v[u]);
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int k = 0; k < V; k++) acc[k].add(v[u][k], (int)(i + u * step + k));
+        fold4<C, OP, V>(acc, v, i, step, 1);
         full += U;
     }
     for (; i < count; i += step) {

@@ -31,15 +31,19 @@ def _ints(shape, dt, seed):
 
 
 def _check_var(G, xs, dt, axis):
-    """The deviations are summed in double (relative error below n 2^-53 of the
-    result, n at most 3e5), the result is rounded to the output type once."""
+    """float64: Welford's updates, a few roundings of 2^-53 a term that add up
+    like sqrt(n).  The others are summed in double and rounded to float32 once."""
     x = O.from_storage(xs, dt).astype(np.float64)
-    rtol = 1e-10 if dt == O.F64 else 2.0 ** -23
+    # numpy adds a contiguous last axis pairwise, any other one element after
+    # element (3e-13 off the exact variance of 20000 whole numbers)
+    x = x.ravel() if axis is None else np.ascontiguousarray(np.moveaxis(x, axis, -1))
+    n = x.shape[-1]
+    rtol = 16 * 2.0 ** -53 * max(n, 16) ** 0.5 if dt == O.F64 else 2.0 ** -23
     for corr, std in ((0, False), (1, True)):
-        if (x.shape[axis] if axis is not None else x.size) <= corr:
+        if n <= corr:
             continue
         got = np.asarray(G.moments(xs, dt, axis, corr, std), np.float64).ravel()
-        ref = np.atleast_1d(x.std(axis, ddof=corr) if std else x.var(axis, ddof=corr)).ravel()
+        ref = np.atleast_1d(x.std(-1, ddof=corr) if std else x.var(-1, ddof=corr)).ravel()
         assert np.allclose(got, ref, rtol=rtol, atol=0, equal_nan=True), (corr, std)
 
 
@@ -100,6 +104,32 @@ def test_variance_far_from_zero(G):
     x[0, 10:20] = -3e4
     for axis in (0, None):
         _check_var(G, x, O.F32, axis)
+
+
+@pytest.mark.parametrize("shape,axis", [((5000, 70), 0), ((70, 3, 50), 1), ((3, 5, 1), 1), ((257, 129), 0),
+                                        ((200000, 40), 0), ((1100, 5000, 1), 1), ((9001,), None),
+                                        ((4000003,), None)], ids=str)
+def test_float64_variance_is_float64_accurate(G, shape, axis):
+    """Ordinary values, and an outlier in first place (of every column, of the
+    tensor): the error is a few roundings of the result, not of the outlier's
+    square over the spread."""
+    from phptensors import synthetic
+    x = synthetic.normal(shape, 0.5, 1.0, seed=3).astype(np.float64)
+    _check_var(G, x, O.F64, axis)
+    x[0 if axis != 1 else (slice(None), 0)] = 1e6
+    _check_var(G, x, O.F64, axis)
+
+
+@pytest.mark.parametrize("axis", [0, None])
+def test_float64_variance_at_the_ends_of_its_range(G, axis):
+    """One extreme value everywhere has variance 0, finite values whose
+    variance leaves float64 have variance inf."""
+    for n in (3, 4, 17, 300, 5000):
+        for v in (np.finfo(np.float64).max, -np.finfo(np.float64).max):
+            assert np.all(np.asarray(G.moments(np.full((n, 5), v), O.F64, axis)) == 0.0)
+        x = np.full((n, 5), 1e200)
+        x[n // 2] = -1e200
+        assert np.all(np.asarray(G.moments(x, O.F64, axis)) == np.inf)
 
 
 def test_global_reduction_of_an_offset_view(G):
