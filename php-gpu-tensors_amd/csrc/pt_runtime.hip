@@ -3,6 +3,7 @@
 // graph capture.  Replaces src/cuda_wrapper.cpp, src/backends/cuda/
 // memory_pool.c and the driver-API calls of src/fusion_*.c /
 // src/compiler_ce.c in the reference.
+#include "pt_blocks.h"
 #include "pt_common.h"
 
 #include <hip/hiprtc.h>
@@ -115,8 +116,8 @@ hipStream_t stream_of(pt_stream_t s)
 //    driver's pool as it is. Any thread may free or take one: whatever a
 //    thread queues after taking a block follows what was queued before the
 //    free on the same stream.
-//  * Sizes are rounded up to an eighth of their power of two (at least 512
-//    bytes), and a block serves its own rounded size only.
+//  * Sizes are rounded up by block_class, and a block serves its own rounded
+//    size only.
 //  * At most kKeepBytes are kept (or the threshold given to pt_mem_init);
 //    a free that would pass it gives every kept block back first.  They are
 //    also given back when an allocation fails.
@@ -131,13 +132,6 @@ static KeptBlocks &kept_blocks()
 {
     static KeptBlocks *k = new KeptBlocks;  // outlives every object freed at process end
     return *k;
-}
-
-static size_t block_class(size_t bytes)
-{
-    size_t step = 512;
-    while (step * 16 <= bytes) step *= 2;
-    return (bytes + step - 1) / step * step;
 }
 
 static bool is_capturing(hipStream_t s)
@@ -162,6 +156,7 @@ static void give_back(KeptBlocks &k)
 
 static hipError_t pool_alloc(void **ptr, size_t bytes, hipStream_t stream)
 {
+    if (bytes > kMaxBlockBytes) return hipErrorOutOfMemory;
     KeptBlocks &k = kept_blocks();
     const bool ours = stream == g_stream && !is_capturing(stream);
     const size_t size = block_class(bytes);

@@ -104,6 +104,21 @@ def test_bound(lib):
     A.check(lib.pt_mem_init(0))
 
 
+@pytest.mark.parametrize("nbytes", [2 ** 63, 2 ** 63 + 1, 2 ** 64 - 512, 2 ** 64 - 1])
+def test_sizes_that_cannot_exist_are_refused(lib, nbytes):
+    p = ctypes.c_void_p()
+    assert lib.pt_alloc(ctypes.byref(p), nbytes, None) == A.PT_ERR_NOMEM and not p.value
+    A.check(lib.pt_free(_alloc(lib, 1000), None))
+
+
+@pytest.mark.parametrize("shape", [(2000000000, 2000000000)], ids=str)
+def test_tensors_that_cannot_exist_are_refused(lib, shape):
+    from phptensors import CudaArray
+    with pytest.raises(A.RuntimeException, match="allocation"):
+        CudaArray.zeros(list(shape))
+    assert CudaArray.full([3], 2.0).toNumpy().tolist() == [2.0] * 3
+
+
 def test_threads_share_the_stream(lib):
     from phptensors import CudaArray
     errors = []
