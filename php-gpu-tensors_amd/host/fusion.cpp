@@ -1936,7 +1936,7 @@ static bool prepare_values(Plan &p, std::vector<TensorP> &vals)
 {
     auto give = [&](int id) {
         const Tensor &t = *p.items[id].t;
-        auto st = buffer_for(p, id, t.numel() * dtype_size(t.dtype));
+        auto st = buffer_for(p, id, storage_bytes(t));
         if (!st) return false;
         TensorP v = make_meta(t.shape, t.ndims, t.dtype);
         if (!v) return false;

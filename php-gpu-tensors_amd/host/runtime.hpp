@@ -104,6 +104,8 @@ bool matmul_shape(const int *a, int na, const int *b, int nb, int *out, int *nou
 
 TensorP make_empty(const int *shape, int ndims, int dtype);  // allocated, uninitialised
 TensorP make_meta(const int *shape, int ndims, int dtype);   // metadata only (lazy)
+// bytes of a contiguous tensor; SIZE_MAX, which no allocation serves, where they overflow
+size_t storage_bytes(const Tensor &t);
 TensorP from_host(const void *data, const int *shape, int ndims, int dtype);
 bool to_host(const TensorP &t, void *out, size_t bytes);     // logical row-major bytes
 TensorP full(const int *shape, int ndims, int dtype, const Scalar &value);

@@ -410,6 +410,12 @@ Storage::~Storage()
     if (ptr) pt_free(ptr, nullptr);
 }
 
+size_t storage_bytes(const Tensor &t)
+{
+    size_t bytes;
+    return __builtin_mul_overflow(t.numel(), dtype_size(t.dtype), &bytes) ? SIZE_MAX : bytes;
+}
+
 static std::atomic<uint64_t> g_ids{1};
 uint64_t next_tensor_id() { return g_ids.fetch_add(1); }
 
@@ -485,7 +491,7 @@ TensorP make_empty(const int *shape, int ndims, int dtype)
     TensorP t = make_meta(shape, ndims, dtype);
     if (!t) return nullptr;
     auto st = std::make_shared<Storage>();
-    size_t bytes = t->numel() * dtype_size(dtype);
+    size_t bytes = storage_bytes(*t);
     st->bytes = bytes;
     if (!check_status(pt_alloc(&st->ptr, bytes ? bytes : 1, nullptr), "device allocation")) return nullptr;
     t->storage = st;

@@ -111,8 +111,10 @@ def test_sizes_that_cannot_exist_are_refused(lib, nbytes):
     A.check(lib.pt_free(_alloc(lib, 1000), None))
 
 
-@pytest.mark.parametrize("shape", [(2000000000, 2000000000)], ids=str)
+@pytest.mark.parametrize("shape", [(2000000000, 2000000000), (65536, 65536, 65536, 16384), (65536, 65536, 65536, 16385)],
+                         ids=str)
 def test_tensors_that_cannot_exist_are_refused(lib, shape):
+    """16 EB, and bytes that wrap to 0 and to 1 PiB in 64 bits."""
     from phptensors import CudaArray
     with pytest.raises(A.RuntimeException, match="allocation"):
         CudaArray.zeros(list(shape))
