@@ -1274,7 +1274,6 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         }
     }
     const bool f32ring = dtype == PT_FLOAT32 && tile == TILE_F32_RING && gemm_f32r_eligible(g, a_kc, b_kc);
-    const bool ktail = g.K % 16 != 0;  // the ring's element-wise tail
     switch (dtype) {
     case PT_BFLOAT16: launch_dt<PT_BFLOAT16>(g, tile, a_kc, b_kc, check, s); break;
     case PT_FLOAT16: launch_dt<PT_FLOAT16>(g, tile, a_kc, b_kc, check, s); break;
@@ -1303,14 +1302,14 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
         PT_TRY(check_hip(e2, "matmul (split-K sum)"));
         counters().mfma_gemm_calls++;
         snprintf(counters().last_matmul, sizeof(counters().last_matmul), "%s%s",
-                 f32ring ? (ktail ? "mfma-fp32-tail-splitk" : "mfma-fp32-ring-splitk") : dtype == PT_FLOAT32 ? "mfma-fp32-splitk" : "mfma-low-precision-splitk",
+                 f32ring ? "mfma-fp32-ring-splitk" : dtype == PT_FLOAT32 ? "mfma-fp32-splitk" : "mfma-low-precision-splitk",
                  suffix);
         return PT_OK;
     }
     PT_LAUNCH_CHECK("matmul");
     counters().mfma_gemm_calls++;
     snprintf(counters().last_matmul, sizeof(counters().last_matmul), "%s%s",
-             f32ring ? (ktail ? "mfma-fp32-tail" : "mfma-fp32-ring") : dtype == PT_FLOAT32 ? "mfma-fp32" : "mfma-low-precision", suffix);
+             f32ring ? "mfma-fp32-ring" : dtype == PT_FLOAT32 ? "mfma-fp32" : "mfma-low-precision", suffix);
     return PT_OK;
 }
 

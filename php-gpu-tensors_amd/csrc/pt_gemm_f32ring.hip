@@ -130,7 +130,8 @@ __global__ __launch_bounds__(256, NST == 2 ? 2 : 1) void k_gemm_f32r(GemmArgs g)
     const long long stb = (B_KC ? (long long)BK : (long long)BK * g.b_sk) * 4;
     // a K chunk may end within its last 32-k step: that step's loads reach
     // past the chunk, and the loads of each step may read only up to the
-    // operand's last element (the buffer unit returns zeros past it)
+    // operand's last element (the buffer unit returns zeros past it, dword by
+    // dword: a last pack that straddles the end keeps its own elements)
     const int KT = (Kl + BK - 1) / BK;
     // TAIL (K not a multiple of 32): the step that ends past the chunk (-1:
     // none), compared as a uniform integer so that the check

@@ -153,11 +153,10 @@ def test_matmul_split_k(A, bmnk, dt):
 
 def _ring_eligible(m, n, k, layout):
     """The fp32 ring kernel's conditions (pt_gemm_f32ring.hip) for these
-    aligned, packed operands: K a multiple of 16 (a last half step of 32 is
-    zero-filled), and a transposed (m- or n-contiguous) operand needs its M
-    or N a multiple of 4."""
-    a_rc, b_rc = layout[0] == "T", layout[1] == "N"
-    return k % 16 == 0 and (not a_rc or m % 4 == 0) and (not b_rc or n % 4 == 0)
+    aligned, contiguous operands: rows of whole 16-byte packs, K a multiple
+    of 4 for a k-contiguous operand, M or N for an m- or n-contiguous one
+    (any K then: the elements of the last 32-k step past it are zeroed)."""
+    return (m if layout[0] == "T" else k) % 4 == 0 and (n if layout[1] == "N" else k) % 4 == 0
 
 
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
@@ -174,9 +173,9 @@ def test_matmul_fp32_ring(A, bmnk, layout):
     where the loads past the operand's end read zeros and the half step's
     upper slices are zeroed.  Integer-valued operands keep every sum exact,
     so outputs are bit-exact against numpy's float64 product.  Shapes the
-    kernel does not take (K % 16 != 0, a transposed operand whose M or N is
-    not a multiple of 4) run the 8-wave 128x128 kernel instead and must
-    agree too."""
+    kernel does not take (rows of no whole 16-byte packs: K no multiple of 4
+    and an operand k-contiguous, or M or N none and an operand transposed) run
+    the 8-wave 128x128 kernel instead and must agree too."""
     from phptensors import synthetic
     b_, m, n, k = bmnk
     A.load().pt_matmul_set_tile(38)

@@ -1,7 +1,8 @@
 """GPU parity of the products at sizes that fill no whole tiles, K steps or
 16-byte packs: integer-valued operands, so that every order of summation gives
 the same bits, against the float64 product; every operand layout, contiguous
-and inside wider arrays, with NaN in the memory that a tail must not use."""
+and inside wider arrays, with NaN in the memory that a tail must not use: rows
+at any element (the register-staged kernels) and aligned ones (the fp32 ring)."""
 import numpy as np
 import pytest
 
@@ -47,6 +48,58 @@ def test_fp32_k_tails(ta, tb, k):
         _check(O.F32, (b, m, n, k), ta, tb, 0)
     _check(O.F32, (1, 128, 132, 4 * k + 2048), ta, tb, 0)
     _check(O.F32, (1, 128, 128, k), ta, tb, 4)
+
+
+def _padded(shape, transposed, before, seed):
+    """Integer values inside an array whose pitch is the next multiple of 4
+    after `before` + the row, at column `before` (0 or 4: packs stay aligned),
+    NaN in every other element; the array ends with the last row's last
+    element.  Returns the values and the array's memory, base, pitch."""
+    from phptensors import synthetic
+    x = synthetic.integers(shape, -4, 5, seed=seed).astype(np.float32)
+    m = np.ascontiguousarray(x.T) if transposed else x
+    pitch = (before + m.shape[1] + 4) // 4 * 4
+    w = np.full((m.shape[0], pitch), np.nan, np.float32)
+    w[:, before:before + m.shape[1]] = m
+    return x, w.ravel()[:(m.shape[0] - 1) * pitch + before + m.shape[1]], before, pitch
+
+
+@pytest.mark.parametrize("ta", [False, True], ids=["A", "At"])
+@pytest.mark.parametrize("tb", [False, True], ids=["B", "Bt"])
+@pytest.mark.parametrize("before", [0, 4])
+@pytest.mark.parametrize("k", [2, 3, 5, 29, 30, 31, 33, 63, 69, 98, 125, 126, 127])
+def test_fp32_ring_beside_nan(ta, tb, before, k):
+    """The ring kernel's K tail in operands of aligned, padded rows: every
+    remainder of K, in a k-contiguous operand the last pack straddles the end
+    of K (and of the array in the last row), and what lies past K is NaN."""
+    from phptensors import _abi as A
+    lib = A.load()
+    A.check(lib.pt_init(), "init")
+    for m, n in ((128, 128), (132, 260)):
+        x, xm, xo, xp = _padded((m, k), ta, before, m + k)
+        y, ym, yo, yp = _padded((k, n), tb, before, n + k)
+        da, db, dc = A.to_device(xm), A.to_device(ym), A.DeviceBuffer(4 * m * n)
+        A.matmul(da.ptr + 4 * xo, db.ptr + 4 * yo, dc.ptr, A.FLOAT32, (m, k), [1, xp] if ta else [xp, 1],
+                 (k, n), [1, yp] if tb else [yp, 1], (m, n))
+        assert A.backend_info().last_matmul.decode() == "mfma-fp32-ring"
+        assert np.array_equal(dc.download(np.float32, (m, n)), (x.astype(np.float64) @ y.astype(np.float64)))
+
+
+@pytest.mark.parametrize("k", [777, 1002])
+def test_fp32_ring_beside_nan_on_a_full_grid(k):
+    """The same where the tiles alone fill the CUs, as columns of wider tensors."""
+    from phptensors import CudaArray, _abi, synthetic
+    m, n = 2052, 2050
+    x = synthetic.integers((m, k), -4, 5, seed=1).astype(np.float32)
+    y = synthetic.integers((n, k), -4, 5, seed=2).astype(np.float32)
+    wide = []
+    for v in (x, y):
+        w = np.full((v.shape[0], 1008), np.nan, np.float32)
+        w[:, 4:4 + k] = v
+        wide.append(CudaArray.fromNumpy(w).slice(":", [4, 4 + k]))
+    got = wide[0].matmul(wide[1].T).toNumpy()
+    assert _abi.backend_info().last_matmul.decode() == "mfma-fp32-ring"
+    assert np.array_equal(got, x.astype(np.float64) @ y.astype(np.float64).T)
 
 
 @pytest.mark.parametrize("dt", list(NAMES), ids=NAMES.get)
