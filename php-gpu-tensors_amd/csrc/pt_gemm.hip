@@ -1011,6 +1011,44 @@ pt_status pt_matmul_set_schedule(int sched)
     return PT_OK;
 }
 
+// Tile of a 16-bit product of t128 tiles of 128x128 that takes neither the
+// ring nor the direct kernel; `kc` of its operands are k-contiguous (the
+// others are transposed on their way into LDS).  Every line lies where the
+// measurements cross (bf16, us).
+//  * Fewer than 256 tiles: 128x128 tiles split K over the CUs (for K of 256
+//    and more), at the price of fp32 partials and a sum; 64x64 tiles fill the
+//    CUs at once.  64x64 against 128x128, by tiles and kc:
+//      16 to 64 tiles: 1024 x 1024 at K 512 / 1024, kc 2 6.9/9.8 against
+//      16.6/22.0, kc 0 11.8/19.8 against 18.2/22.9; at K 2048 ahead only up to
+//      32 tiles (512 x 1024, kc 0 21.1 against 22.2);
+//      144: kc 2 K 1024 16.2 against 22.2, kc 1 23.4 against 23.7, kc 0 K 640
+//      22.3 against 25.1, K 768 25.9 against 25.5, K 1024 32.2 against 25.9;
+//      240: kc 2 K 1024 21.7 against 26.2, kc 1 K 896 26.7 against 27.5, K 1024
+//      29.3 against 28.7, kc 0 K 640 27.9 against 28.1, K 768 32.1 against 29.0.
+//  * From 256 tiles on nothing is split.  Four waves against eight:
+//      256 (2048 x 2048): kc 2 K 1024 18.8 against 16.9, kc 1 23.7 against
+//      22.6, kc 0 29.7 against 28.8, K 2000 56.1 against 62.5;
+//      512 (4096 x 2048): kc 2 K 512 19.0 against 17.4, kc 1 K 128 11.9
+//      against 11.8, K 512 21.2 against 22.2, K 1024 32.9 against 35.7, kc 0
+//      K 64 about equal, K 128 12.9 against 13.8, K 1024 40.0 against 46.4;
+//      more than 512: kc 1 K 512 42.0 against 38.4 (12 x 1000 x 1001), 30.6
+//      against 30.5 (20 x 1024 x 512) and 75.5 against 79.2 (28 x 1000 x 1000),
+//      K 1024 47.8 against 50.1 (20 x 1024 x 512), kc 0 K 128 19.1 against
+//      18.5, K 384 30.1 against 31.6;
+//      280 to 384: kc 2 K 2048 equal, K 4096 77.5 against 82.5.
+static int half_tile(long long t128, long long K, int kc)
+{
+    if (t128 < 256) {
+        const long long most = t128 <= 32 ? 2048 : t128 <= 128 ? 1024 : kc == 2 ? 1024 : kc == 0 ? 640 : t128 <= 192 ? 1024 : 896;
+        return K <= most ? TILE_64x64 : TILE_128x128;
+    }
+    const long long most = kc == 2         ? 2048
+                           : t128 == 256   ? (kc ? 2048 : 1024)
+                           : t128 <= 512   ? (kc ? 128 : 64)
+                                           : (kc ? 512 : 128);
+    return K <= most ? TILE_128x128_W8 : TILE_128x128;
+}
+
 // Tile override (see kTiles), -1 = automatic.
 pt_status pt_matmul_set_tile(int tile)
 {
@@ -1113,30 +1151,23 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
     const char *suffix = tuned ? "-tuned" : "";
     if (tile < 0) {
         long long t256 = ((g.M + 255) / 256) * (long long)((g.N + 255) / 256) * batch;
-        // Mid-size products.  128x128 tiles of 8 waves where they give every
-        // CU one: fp32 for either layout of B (dZ2 W2^T of config 5, B
-        // k-contiguous: 76-78 us against 82-84 us for 128x64 tiles at two
-        // workgroups per CU), 16-bit 12 x 1000 x 1001 x 777 fp16 43.5 us
-        // against 52 us with 4 waves, 2048^3 bf16 34.8 against 37.0.
-        // Fewer tiles split K over the CUs, at the price of fp32 partials
-        // and a sum, which pays only over a long K (there 4 waves stay ahead
-        // for 16 bits); below it 64x64 tiles fill the CUs at once.  64x64
-        // against split 128x128, bf16, us, by K 256 / 512 / 1024 / 2048:
-        // 1024 x 1024 6.8/9.8/13.6/23.5 against 13.5/17.2/21.7/21.9,
-        // 512 x 512 (16 tiles) 13.5 against 17.2 at K 2048.  fp32 keeps the
-        // split (1024 x 1024 9.9/14.6/26.6/56.0 against 18.9/24.4/27.7/40.4):
-        // another order of its sums moves single ReLU decisions of a training
-        // step, whose gradients then differ by more than rounding.
+        // Mid-size products: 128x128 tiles where they give every CU one
+        // (half_tile chooses their waves for 16 bits; fp32 8 waves for either
+        // layout of B: dZ2 W2^T of config 5, B k-contiguous, 76-78 us against
+        // 82-84 us for 128x64 tiles at two workgroups per CU), else half_tile
+        // chooses between splitting their K and 64x64 tiles.  fp32 keeps the
+        // split (1024 x 1024 by K 256 / 512 / 1024 / 2048: 64x64 tiles
+        // 9.9/14.6/26.6/56.0 us against 18.9/24.4/27.7/40.4): another order
+        // of its sums moves single ReLU decisions of a training step, whose
+        // gradients then differ by more than rounding.
         const long long t128 = ((g.M + 127) / 128) * (long long)((g.N + 127) / 128) * batch;
-        const bool f32 = dtype == PT_FLOAT32;
-        const bool narrow = !f32 && t128 < 256 && (g.K <= 1024 || (g.K <= 2048 && t128 <= 32));
         tile = (g.M >= 256 && g.N >= 256 && t256 >= 256)
-                   ? (f32 ? TILE_256x256
+                   ? (dtype == PT_FLOAT32 ? TILE_256x256
                       : g.K % 64 != 0 ? TILE_RING_HALF
                       : dtype == PT_BFLOAT16 ? TILE_RING_DEFAULT : TILE_RING_DEFAULT_F16)
-               : g.M < 128 || g.N < 128 || narrow ? TILE_64x64
-               : f32 || t128 >= 256               ? TILE_128x128_W8
-                                                  : TILE_128x128;
+               : g.M < 128 || g.N < 128 ? TILE_64x64
+               : dtype == PT_FLOAT32    ? TILE_128x128_W8
+                                        : half_tile(t128, g.K, (a_kc ? 1 : 0) + (b_kc ? 1 : 0));
     }
     // the fp32-only tiles run the 128x128 kernel for 16-bit operands
     if (dtype != PT_FLOAT32 && (tile == TILE_128x128_W8_K2 || tile == TILE_128x64_W4M2 || tile == TILE_128x64_W4M2_K2 ||

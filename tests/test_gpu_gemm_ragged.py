@@ -123,6 +123,19 @@ def test_ragged_split_k_and_large_tiles(dt, ta, tb):
     _check(dt, (9, 1300, 1291, 70), ta, tb, 0)  # 256x256 tiles
 
 
+@pytest.mark.parametrize("dt", [O.BF16, O.F16], ids=NAMES.get)
+@pytest.mark.parametrize("ta", [False, True], ids=["A", "At"])
+@pytest.mark.parametrize("tb", [False, True], ids=["B", "Bt"])
+@pytest.mark.parametrize("bmn,ks", [((1, 510, 1024), (2048, 2050)), ((1, 1150, 2046), (640, 641, 1024, 1025)),
+                                    ((2, 900, 1500), (640, 641, 896, 897, 1024)), ((1, 2048, 2046), (1024, 1025)),
+                                    ((5, 900, 850), (64, 65, 128, 129)), ((13, 900, 850), (128, 129, 512, 513))],
+                         ids=str)
+def test_both_sides_of_the_16_bit_tile_rule(dt, ta, tb, bmn, ks):
+    """64x64 tiles, 128x128 tiles with K split, of four waves and of eight, by number of tiles, K and layout."""
+    for k in ks:
+        _check(dt, bmn + (k,), ta, tb, 0)
+
+
 @pytest.mark.parametrize("dt", list(NAMES), ids=NAMES.get)
 def test_nonfinite_operands_stay_in_their_rows(dt):
     """Infinities and NaN next to a K tail reach exactly the outputs whose sums hold them."""
