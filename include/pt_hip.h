@@ -116,6 +116,11 @@ pt_status pt_device_synchronize(void);
 const char *pt_status_string(pt_status status);
 const char *pt_last_error(void);
 pt_status pt_version(int *major, int *minor);
+/* 1 when the process has one HIP runtime mapped and it is of the version
+ * (major.minor) this library was built against; 0 when another library (a
+ * PyTorch wheel, say) brought its own, which then serves this library too
+ * where it was loaded first.  Needs no device. */
+int pt_runtime_is_own(void);
 
 /* --------------------------------------------------------------- streams --
  * The reference's Fusion executor creates private non-blocking streams and

@@ -9,6 +9,8 @@
 #include <hip/hiprtc.h>
 
 #include <algorithm>
+#include <atomic>
+#include <link.h>
 #include <mutex>
 #include <stdarg.h>
 #include <stdio.h>
@@ -395,6 +397,42 @@ pt_status pt_version(int *major, int *minor)
     if (major) *major = 0;
     if (minor) *minor = 1;
     return PT_OK;
+}
+
+// Objects mapped into the process: the loader's count of loads so far and,
+// when asked for, the HIP runtimes among them.
+struct MappedRuntimes {
+    unsigned long long loads = 0;
+    int runtimes = 0;
+    bool count = true;
+};
+static int mapped_object(struct dl_phdr_info *info, size_t, void *arg)
+{
+    MappedRuntimes *m = (MappedRuntimes *)arg;
+    m->loads = info->dlpi_adds;
+    if (!m->count) return 1;
+    const char *slash = strrchr(info->dlpi_name, '/');
+    if (strncmp(slash ? slash + 1 : info->dlpi_name, "libamdhip64.so", 14) == 0) m->runtimes++;
+    return 0;
+}
+
+int pt_runtime_is_own(void)
+{
+    // asked before each execution of a captured plan: the objects are walked
+    // again only after the loader has loaded another one
+    static std::atomic<unsigned long long> seen{0};  // loads at the last walk, times 2, plus its answer
+    MappedRuntimes m;
+    m.count = false;
+    dl_iterate_phdr(mapped_object, &m);
+    const unsigned long long last = seen.load();
+    if (last && last >> 1 == m.loads) return (int)(last & 1);
+    m = MappedRuntimes();
+    dl_iterate_phdr(mapped_object, &m);
+    int version = 0;
+    const bool same = hipRuntimeGetVersion(&version) == hipSuccess && version / 100000 == HIP_VERSION / 100000;
+    const int own = same && m.runtimes == 1;
+    seen.store(m.loads << 1 | (unsigned)own);
+    return own;
 }
 
 pt_status pt_device_count(int *count)

@@ -1595,6 +1595,20 @@ static Plan *build_plan(const std::vector<TensorP> &roots, const std::vector<Ten
 }
 
 // ------------------------------------------------------------ execution
+// Plans of several steps are captured over several streams only on the HIP
+// runtime this library was built with: on another one (a process that loads
+// a PyTorch wheel first runs on the wheel's) the capture of the training
+// step ended in a host segmentation fault.  The branch code keeps every rule
+// of stream capture (each event recorded before it is waited on and alive
+// until the capture has ended, each stream joined), so the fault is taken to
+// be that runtime's, and such plans run step by step.
+static void settle_graph(Plan &p)
+{
+    if (!p.use_graph || !p.graph_compatible || p.steps.size() < 2 || pt_runtime_is_own()) return;
+    p.graph_compatible = false;
+    p.incompatibility = "foreign-hip-runtime";
+}
+
 static uint64_t now_ns()
 {
     struct timespec ts;
@@ -2126,6 +2140,7 @@ static bool execute(Plan &p, const std::vector<TensorP> &inputs, std::vector<Ten
     }
     if (!prepare_values(p, vals)) return false;
     uint64_t t1 = now_ns();
+    settle_graph(p);
     bool graph_ok = p.use_graph && p.graph_compatible;
     bool native_present = false;
     for (Step &st : p.steps) native_present = native_present || st.native;
@@ -2364,6 +2379,7 @@ phpt_graph *phpt_fusion_end(phpt_tensor **outputs, int count, int use_graph)
         delete p;
         return nullptr;
     }
+    settle_graph(*p);
     auto *g = new phpt_graph;
     g->plan = p;
     return g;
@@ -2579,7 +2595,7 @@ const char *phpt_graph_stats(phpt_graph *g)
        << ";cudaGraphIncompatibility="
        << (p.graph_compatible ? "null" : p.incompatibility ? p.incompatibility : "native-graph-not-supported")
        << ";incompatibility=" << (p.incompatibility ? p.incompatibility : "null")
-       << ";graphReplay=" << (p.use_graph && !native_present ? 1 : 0)
+       << ";graphReplay=" << (p.use_graph && p.graph_compatible && !native_present ? 1 : 0)
        << ";graphLaunches=" << p.graph_launches << ";bufferReuses=" << p.buffer_reuses
        << ";pending=" << p.pending << ";cudaGraphRequested=" << (p.use_graph ? 1 : 0)
        << ";tensorAllocations=" << p.tensor_allocations << ";synchronizations=" << p.synchronizations

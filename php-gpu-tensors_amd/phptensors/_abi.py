@@ -76,6 +76,7 @@ SIGNATURES = {
     "pt_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "pt_last_error": (ctypes.c_char_p, []),
     "pt_version": (ctypes.c_int, [c_int_p, c_int_p]),
+    "pt_runtime_is_own": (ctypes.c_int, []),
     "pt_stream_create": (ctypes.c_int, [ctypes.POINTER(vp)]),
     "pt_stream_destroy": (ctypes.c_int, [vp]),
     "pt_stream_synchronize": (ctypes.c_int, [vp]),
