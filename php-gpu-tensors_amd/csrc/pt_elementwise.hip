@@ -716,19 +716,25 @@ static unsigned opnd_cols(const EwShape &s)
     return c > 0x7fffffffLL ? 1u : (unsigned)c;  // only read where an operand is rowwise (at most 2^31 elements)
 }
 
-// Streaming accesses bypass cache retention (nontemporal) in calls that move
-// a gigabyte or more through aligned chunks: the 256 MB Infinity Cache then
-// holds nothing that the next call could read.  A chain of eager calls (add,
-// gt, where, multiply, add, astype; cached against nontemporal):
-// [8000, 3001] bf16 150 against 166 us, [8000, 3000] fp32 201 against 215,
-// [16000, 8000] bf16 (0.77 GB a call) 690 against 735, [16000, 8001] fp32
-// (1.5 GB a call) 1050 against 992, and tanh of [16384, 8192] fp32 (1.07 GB)
-// 175 against 165.
-static bool streams(size_t bytes, std::initializer_list<const void *> ptrs)
+// Streaming accesses bypass cache retention (nontemporal) in calls through
+// aligned chunks that move `least` bytes or more.  Ordinarily a gigabyte: the
+// 256 MB Infinity Cache then holds nothing that the next call could read.  A
+// chain of eager calls (add, gt, where, multiply, add, astype; cached against
+// nontemporal): [8000, 3001] bf16 150 against 166 us, [8000, 3000] fp32 201
+// against 215, [16000, 8001] fp32 (1.5 GB a call) 1050 against 992, and tanh
+// of [16384, 8192] fp32 (1.07 GB) 175 against 165.
+// Calls on two full operands stream from 256 MB on: with the output they are
+// three streams that do not fit the cache together, and what they evict is
+// the result of the call before.  x + m of [8192, 4096] fp32 (403 MB) 69.4
+// cached and 62.6 us nontemporal, y * x, + m and tanh of it 150 and 137, of
+// [8192, 8192] 314 and 285, of [16000, 8000] bf16 328 and 302; the six calls
+// of [4096, 4096] fp32 (201 MB a sum) 147 and 150.
+constexpr size_t kStreamBytes = 1000000000, kStreamPairBytes = (size_t)256 << 20;
+static bool streams(size_t bytes, size_t least, std::initializer_list<const void *> ptrs)
 {
     for (const void *p : ptrs)
         if ((uintptr_t)p & 15) return false;
-    return bytes >= 1000000000;
+    return bytes >= least;
 }
 
 static bool vec_float(int dt) { return dt == PT_FLOAT32 || dt == PT_FLOAT16 || dt == PT_BFLOAT16; }
@@ -773,7 +779,9 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
     if (vec) {
         if (reverse) std::swap(oa, ob);
         const size_t total = (size_t)s.total;
+        const bool pair = oa.mode == OPND_FLAT && ob.mode == OPND_FLAT;
         const bool nt = streams(total * (dtype_size(dta) * (scalar ? 1 : 2) + dtype_size(dto)),
+                                pair ? kStreamPairBytes : kStreamBytes,
                                 {oa.mode == OPND_FLAT ? oa.p : nullptr, ob.mode == OPND_FLAT ? ob.p : nullptr, out});
         with_vec_dtype(dta, [&](auto D) {
             constexpr int DT = decltype(D)::value;
@@ -792,7 +800,7 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
             using RW = std::integral_constant<int, OPND_ROWS>;
             using AN = std::integral_constant<int, OPND_ANY>;
             if (dto != dta) go(std::integral_constant<int, PT_FLOAT32>{}, AN{}, AN{});
-            else if (oa.mode == OPND_FLAT && ob.mode == OPND_FLAT) go(D, FL{}, FL{});
+            else if (pair) go(D, FL{}, FL{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_IMM) go(D, FL{}, IM{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_ROWS) go(D, FL{}, RW{});
             else if (oa.mode == OPND_ROWS && ob.mode == OPND_FLAT) go(D, RW{}, FL{});
@@ -860,7 +868,7 @@ pt_status pt_unary(const void *input, int dtype, const size_t *strides, size_t o
     Opnd ox;
     if (vec_float(dtype) && as_opnd(s, s.sa, px, ox)) {
         const size_t total = (size_t)s.total;
-        const bool nt = streams(total * dtype_size(dtype) * 2, {ox.mode == OPND_FLAT ? px : nullptr, out});
+        const bool nt = streams(total * dtype_size(dtype) * 2, kStreamBytes, {ox.mode == OPND_FLAT ? px : nullptr, out});
         with_vec_dtype(dtype, [&](auto D) {
             constexpr int DT = decltype(D)::value;
             const unsigned grid = grid_for(s.total, 16 / (int)sizeof(typename VecT<DT>::T)), cols = opnd_cols(s);
@@ -922,7 +930,7 @@ pt_status pt_cast(const void *input, int dtype_in, const size_t *strides, size_t
     EwShape32 s32;
     if (vec_float(dtype_in) && vec_float(dtype_out) && dtype_in != dtype_out && as_opnd(s, s.sa, px, ox)) {
         const size_t total = (size_t)s.total;
-        const bool nt = streams(total * (dtype_size(dtype_in) + dtype_size(dtype_out)),
+        const bool nt = streams(total * (dtype_size(dtype_in) + dtype_size(dtype_out)), kStreamBytes,
                                 {ox.mode == OPND_FLAT ? px : nullptr, out});
         with_vec_dtype(dtype_in, [&](auto I) {
             with_vec_dtype(dtype_out, [&](auto O) {
@@ -961,7 +969,7 @@ pt_status pt_where(const void *cond, int dtype_cond, const size_t *strides_cond,
         const size_t total = (size_t)s.total;
         // a floating condition holds unless it is +0 or -0; integers and bool unless they are 0
         const uint32_t mask = dtype_is_floating(dtype_cond) ? (csz == 4 ? 0x7fffffffu : 0x7fffu) : 0xffffffffu;
-        const bool nt = streams(total * (size_t)(csz + 3 * esz),
+        const bool nt = streams(total * (size_t)(csz + 3 * esz), kStreamBytes,
                                 {oc.mode == OPND_FLAT ? cond : nullptr, ox.mode == OPND_FLAT ? x : nullptr,
                                  oy.mode == OPND_FLAT ? y : nullptr, out});
         auto go = [&](auto E, auto C, auto N) {
