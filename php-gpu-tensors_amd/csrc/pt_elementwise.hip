@@ -794,16 +794,20 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
             // the layouts of most calls have kernels of their own: y * z of
             // a row and [16384, 8192] fp32 took 181 us with the layouts read
             // at run time (two branches before the loads) against 169.5
-            // (177 with the contiguous operand loaded before the row)
+            // (177 with the contiguous operand loaded before the row), one
+            // value per row (x * c) 184 against 166
             using FL = std::integral_constant<int, OPND_FLAT>;
             using IM = std::integral_constant<int, OPND_IMM>;
             using RW = std::integral_constant<int, OPND_ROWS>;
+            using CL = std::integral_constant<int, OPND_COL>;
             using AN = std::integral_constant<int, OPND_ANY>;
             if (dto != dta) go(std::integral_constant<int, PT_FLOAT32>{}, AN{}, AN{});
             else if (pair) go(D, FL{}, FL{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_IMM) go(D, FL{}, IM{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_ROWS) go(D, FL{}, RW{});
             else if (oa.mode == OPND_ROWS && ob.mode == OPND_FLAT) go(D, RW{}, FL{});
+            else if (oa.mode == OPND_FLAT && ob.mode == OPND_COL) go(D, FL{}, CL{});
+            else if (oa.mode == OPND_COL && ob.mode == OPND_FLAT) go(D, CL{}, FL{});
             else go(D, AN{}, AN{});
         });
     } else {
