@@ -154,6 +154,10 @@ pt_status pt_mem_init(size_t pool_bytes);
 pt_status pt_alloc(void **ptr, size_t bytes, pt_stream_t stream);
 pt_status pt_free(void *ptr, pt_stream_t stream);
 pt_status pt_mem_info(size_t *free_bytes, size_t *total_bytes, size_t *pool_reserved);
+/* Freed blocks that the library keeps for the runtime stream's next
+ * allocations of the same size (part of pool_reserved): at most 8 GiB, or
+ * pool_bytes of pt_mem_init where that is less. */
+pt_status pt_mem_kept(size_t *bytes, size_t *blocks);
 /* Transfers (replace cudaMemcpy in src/cuda_array/tensor_transfer.c:45-65,
  * src/cuda_array/tensor_factory.c:301-326).  Synchronous w.r.t. the host.
  * A pageable host buffer of 4 MiB or more is moved through the library's

@@ -16,7 +16,6 @@
 #include <stdio.h>
 #include <string.h>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 namespace pt {
@@ -106,36 +105,6 @@ hipStream_t stream_of(pt_stream_t s)
     return s ? (hipStream_t)s : (t_current ? t_current : g_stream);
 }
 
-// Blocks freed on the runtime stream, kept for the next allocations there.
-// A block that is allocated, used and freed in one stream's order can go to
-// that stream's next user without a marker on the GPU or a call into the
-// driver; hipMallocAsync and hipFreeAsync cost 4-5 us of host time each and
-// leave gaps between the kernels around them (an eager add of 64 x 64 took
-// 17.5 us, 6 of them its launch; softmax and layerNorm of [8192, 4096] fp32
-// took 102 us with kernels of 87).
-//  * Only blocks that were allocated and are freed on the runtime stream
-//    while it is not being captured are kept; every other call goes to the
-//    driver's pool as it is. Any thread may free or take one: whatever a
-//    thread queues after taking a block follows what was queued before the
-//    free on the same stream.
-//  * Sizes are rounded up by block_class, and a block serves its own rounded
-//    size only.
-//  * At most kKeepBytes are kept (or the threshold given to pt_mem_init);
-//    a free that would pass it gives every kept block back first.  They are
-//    also given back when an allocation fails.
-static constexpr size_t kKeepBytes = (size_t)8 << 30;
-struct KeptBlocks {
-    std::mutex mu;
-    std::unordered_map<void *, size_t> live;                   // rounded size of blocks handed out
-    std::unordered_map<size_t, std::vector<void *>> kept;      // free blocks by rounded size
-    size_t bytes = 0, limit = kKeepBytes;
-};
-static KeptBlocks &kept_blocks()
-{
-    static KeptBlocks *k = new KeptBlocks;  // outlives every object freed at process end
-    return *k;
-}
-
 static bool is_capturing(hipStream_t s)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -146,75 +115,34 @@ static bool is_capturing(hipStream_t s)
     return st != hipStreamCaptureStatusNone;
 }
 
-// Every kept block back to the driver's pool (the caller holds the lock and
-// the runtime stream is not being captured).
-static void give_back(KeptBlocks &k)
+// The driver's stream-ordered pool, as KeptBlocks uses it.
+struct HipPool {
+    using Stream = hipStream_t;
+    using Status = hipError_t;
+    static constexpr Status kOk = hipSuccess, kNoMemory = hipErrorOutOfMemory;
+    static Status alloc(void **ptr, size_t bytes, Stream s)
+    {
+        const Status st = hipMallocAsync(ptr, bytes, s);
+        if (st != hipSuccess) (void)hipGetLastError();
+        return st;
+    }
+    static Status free(void *ptr, Stream s) { return hipFreeAsync(ptr, s); }
+    static void synchronize(Stream s) { (void)hipStreamSynchronize(s); }
+    static bool capturing(Stream s) { return is_capturing(s); }
+};
+
+static KeptBlocks<HipPool> &kept_blocks()
 {
-    for (auto &c : k.kept)
-        for (void *p : c.second) (void)hipFreeAsync(p, g_stream);
-    k.kept.clear();
-    k.bytes = 0;
+    static KeptBlocks<HipPool> *k = new KeptBlocks<HipPool>;  // outlives every object freed at process end
+    return *k;
 }
 
 static hipError_t pool_alloc(void **ptr, size_t bytes, hipStream_t stream)
 {
-    if (bytes > kMaxBlockBytes) return hipErrorOutOfMemory;
-    KeptBlocks &k = kept_blocks();
-    const bool ours = stream == g_stream && !is_capturing(stream);
-    const size_t size = block_class(bytes);
-    if (ours) {
-        std::lock_guard<std::mutex> lock(k.mu);
-        auto it = k.kept.find(size);
-        if (it != k.kept.end() && !it->second.empty()) {
-            *ptr = it->second.back();
-            it->second.pop_back();
-            k.bytes -= size;
-            k.live[*ptr] = size;
-            return hipSuccess;
-        }
-        hipError_t err = hipMallocAsync(ptr, size, stream);
-        if (err == hipSuccess) {
-            k.live[*ptr] = size;
-            return err;
-        }
-        (void)hipGetLastError();
-        // out of memory: without the kept blocks, and without the rounding
-        give_back(k);
-        (void)hipStreamSynchronize(g_stream);
-        return hipMallocAsync(ptr, bytes, stream);
-    }
-    hipError_t err = hipMallocAsync(ptr, bytes, stream);
-    if (err == hipErrorOutOfMemory && !is_capturing(stream) && !is_capturing(g_stream)) {
-        (void)hipGetLastError();
-        {
-            std::lock_guard<std::mutex> lock(k.mu);
-            give_back(k);
-        }
-        (void)hipStreamSynchronize(g_stream);
-        err = hipMallocAsync(ptr, bytes, stream);
-    }
-    return err;
+    return kept_blocks().alloc(ptr, bytes, stream, g_stream);
 }
 
-static hipError_t pool_free(void *ptr, hipStream_t stream)
-{
-    KeptBlocks &k = kept_blocks();
-    {
-        std::lock_guard<std::mutex> lock(k.mu);
-        auto it = k.live.find(ptr);
-        if (it != k.live.end()) {
-            const size_t size = it->second;
-            k.live.erase(it);
-            if (stream == g_stream && size <= k.limit && !is_capturing(stream)) {
-                if (k.bytes + size > k.limit) give_back(k);
-                k.kept[size].push_back(ptr);
-                k.bytes += size;
-                return hipSuccess;
-            }
-        }
-    }
-    return hipFreeAsync(ptr, stream);
-}
+static hipError_t pool_free(void *ptr, hipStream_t stream) { return kept_blocks().release(ptr, stream, g_stream); }
 
 // Static scratch of the no-allocation entry points (pt_reduce_noalloc): a
 // file-scope device array that every GPU the library runs on holds for the
@@ -577,12 +505,7 @@ pt_status pt_mem_init(size_t pool_bytes)
 {
     PT_TRY(ensure_init());
     uint64_t threshold = pool_bytes ? (uint64_t)pool_bytes : UINT64_MAX;
-    KeptBlocks &k = kept_blocks();
-    {
-        std::lock_guard<std::mutex> lock(k.mu);
-        k.limit = pool_bytes && pool_bytes < kKeepBytes ? pool_bytes : kKeepBytes;
-        if (k.bytes > k.limit && !is_capturing(g_stream)) give_back(k);
-    }
+    kept_blocks().set_limit(pool_bytes, g_stream);
     return check_hip(hipMemPoolSetAttribute(g_pool, hipMemPoolAttrReleaseThreshold, &threshold),
                      "hipMemPoolSetAttribute");
 }
@@ -618,6 +541,13 @@ pt_status pt_mem_info(size_t *free_bytes, size_t *total_bytes, size_t *pool_rese
                          "hipMemPoolGetAttribute"));
         *pool_reserved = (size_t)reserved;
     }
+    return PT_OK;
+}
+
+pt_status pt_mem_kept(size_t *bytes, size_t *blocks)
+{
+    PT_TRY(ensure_init());
+    kept_blocks().usage(bytes, blocks);
     return PT_OK;
 }
 

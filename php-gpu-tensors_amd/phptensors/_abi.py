@@ -91,6 +91,7 @@ SIGNATURES = {
     "pt_event_query": (ctypes.c_int, [vp, c_int_p]),
     "pt_event_elapsed_ms": (ctypes.c_int, [vp, vp, ctypes.POINTER(ctypes.c_float)]),
     "pt_mem_init": (ctypes.c_int, [ctypes.c_size_t]),
+    "pt_mem_kept": (ctypes.c_int, [c_size_p, c_size_p]),
     "pt_alloc": (ctypes.c_int, [ctypes.POINTER(vp), ctypes.c_size_t, vp]),
     "pt_free": (ctypes.c_int, [vp, vp]),
     "pt_mem_info": (ctypes.c_int, [c_size_p, c_size_p, c_size_p]),

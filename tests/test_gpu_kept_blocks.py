@@ -27,6 +27,12 @@ def _alloc(lib, nbytes, stream=None):
     return p.value
 
 
+def _kept(lib):
+    size, count = ctypes.c_size_t(), ctypes.c_size_t()
+    A.check(lib.pt_mem_kept(ctypes.byref(size), ctypes.byref(count)))
+    return size.value, count.value
+
+
 @pytest.mark.parametrize("nbytes", [1, 511, 512, 513, 8191, 8192, 8193, 100000, 1 << 20, (1 << 20) + 1, 50_000_001])
 def test_block_returns_for_its_size_only(lib, nbytes):
     p = _alloc(lib, nbytes)
@@ -57,9 +63,17 @@ def test_other_streams_and_captures_pass_by(lib):
     A.check(lib.pt_stream_create(ctypes.byref(stream)))
     p = _alloc(lib, 70000)
     A.check(lib.pt_stream_synchronize(None))
+    before = _kept(lib)
     A.check(lib.pt_free(p, stream))
+    assert _kept(lib) == before
+    p = _alloc(lib, 70000, stream)
+    A.check(lib.pt_stream_synchronize(stream))
+    A.check(lib.pt_free(p, None))  # allocated on the other stream
+    assert _kept(lib) == before
     q = _alloc(lib, 70000)
+    before = _kept(lib)
     A.check(lib.pt_free(q, None))
+    assert _kept(lib) == (before[0] + 73728, before[1] + 1)
     A.check(lib.pt_stream_synchronize(stream))
     A.check(lib.pt_stream_destroy(stream))
 
@@ -74,9 +88,11 @@ def test_other_streams_and_captures_pass_by(lib):
 
     reduce()
     graph = ctypes.c_void_p()
+    before = _kept(lib)
     A.check(lib.pt_graph_begin_capture(None))
     reduce()
     A.check(lib.pt_graph_end_capture(None, ctypes.byref(graph)))
+    assert _kept(lib) == before
     for i in range(6):
         A.check(lib.pt_memset(out.ptr, 0xFF, 160, None))
         A.check(lib.pt_graph_launch(graph, None))
@@ -92,16 +108,44 @@ def test_other_streams_and_captures_pass_by(lib):
 def test_bound(lib):
     """Blocks beyond the bound go back to the driver's pool, and the bound can be lowered."""
     A.check(lib.pt_mem_init(1 << 20))
+    assert _kept(lib)[0] <= 1 << 20
     blocks = [_alloc(lib, 300_000) for _ in range(8)]
+    assert len(set(blocks)) == 8
     for b in blocks:
         A.check(lib.pt_free(b, None))
+        assert 0 < _kept(lib)[0] <= 1 << 20
+    before = _kept(lib)
     big = _alloc(lib, 8 << 20)  # larger than the bound: not kept
     A.check(lib.pt_free(big, None))
+    assert _kept(lib) == before
     again = [_alloc(lib, 300_000) for _ in range(8)]
-    assert len(set(again)) == 8
-    for b in again:
+    assert len(set(again)) == 8 and _kept(lib) == (before[0] - before[1] * 327680, 0)
+    for b in again[:2]:
+        A.check(lib.pt_free(b, None))
+    assert _kept(lib) == (2 * 327680, 2)
+    A.check(lib.pt_mem_init(400_000))
+    assert _kept(lib) == (0, 0)
+    for b in again[2:]:
         A.check(lib.pt_free(b, None))
     A.check(lib.pt_mem_init(0))
+
+
+def test_failed_allocation_gives_back(lib):
+    """More than the card holds: refused, after every kept block went back to the driver's pool."""
+    total = ctypes.c_size_t()
+    A.check(lib.pt_mem_info(None, ctypes.byref(total), None))
+    stream = ctypes.c_void_p()
+    A.check(lib.pt_stream_create(ctypes.byref(stream)))
+    for st in (None, stream):
+        A.check(lib.pt_free(_alloc(lib, 1 << 20), None))
+        assert _kept(lib)[1] > 0
+        p = ctypes.c_void_p()
+        assert lib.pt_alloc(ctypes.byref(p), 4 * total.value, st) == A.PT_ERR_NOMEM and not p.value
+        assert _kept(lib) == (0, 0)
+        x = A.to_device(np.arange(100, dtype=np.float32))
+        assert np.array_equal(x.download(np.float32, (100,)), np.arange(100))
+        x.free()
+    A.check(lib.pt_stream_destroy(stream))
 
 
 @pytest.mark.parametrize("nbytes", [2 ** 63, 2 ** 63 + 1, 2 ** 64 - 512, 2 ** 64 - 1])
