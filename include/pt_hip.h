@@ -149,14 +149,17 @@ pt_status pt_event_elapsed_ms(pt_event_t start, pt_event_t stop, float *ms);
  * (tensor_mem_init, cuda_mem_alloc, cuda_mem_free) with a stream-ordered
  * HIP memory pool; frees are ordered on the given stream instead of
  * assuming default-stream ordering.  pool_bytes is the retained-memory
- * threshold (INI phptensors.cuda.memory_pool_size, src/cuda.c:64-81). */
+ * threshold (INI phptensors.cuda.memory_pool_size, src/cuda.c:64-81): while
+ * more than that is reserved, freed memory goes back to the device; 0, as
+ * before the first call, sets none. */
 pt_status pt_mem_init(size_t pool_bytes);
 pt_status pt_alloc(void **ptr, size_t bytes, pt_stream_t stream);
 pt_status pt_free(void *ptr, pt_stream_t stream);
 pt_status pt_mem_info(size_t *free_bytes, size_t *total_bytes, size_t *pool_reserved);
 /* Freed blocks that the library keeps for the runtime stream's next
- * allocations of the same size (part of pool_reserved): at most 8 GiB, or
- * pool_bytes of pt_mem_init where that is less. */
+ * allocations of the same size (part of pool_reserved).  At most 8 GiB, and
+ * with the blocks in use there no more than pool_bytes of pt_mem_init; other
+ * streams and other sizes get them when an allocation would fail. */
 pt_status pt_mem_kept(size_t *bytes, size_t *blocks);
 /* Transfers (replace cudaMemcpy in src/cuda_array/tensor_transfer.c:45-65,
  * src/cuda_array/tensor_factory.c:301-326).  Synchronous w.r.t. the host.

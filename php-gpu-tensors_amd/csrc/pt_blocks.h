@@ -39,10 +39,14 @@ inline size_t block_class(size_t bytes)
 //    free on the same stream.
 //  * Sizes are rounded up by block_class, and a block serves its own rounded
 //    size only.
-//  * At most kKeepBytes are kept (or a smaller limit given to set_limit); a
-//    free that would pass it gives every kept block back first.  They are
-//    also given back when an allocation fails, on whatever stream, and the
-//    allocation is then tried once more.
+//  * At most kKeepBytes are kept; a free that would pass it gives every kept
+//    block back first.  They are also given back when an allocation fails, on
+//    whatever stream, and the allocation is then tried once more.
+//  * The driver's pool holds on to freed memory as long as no more than its
+//    threshold is reserved, kept blocks and blocks in use among them.  The
+//    same threshold, where one is set (set_threshold), bounds the home
+//    stream's blocks here: while those in use and those kept come to more,
+//    none are kept.
 template <typename Driver>
 class KeptBlocks {
 public:
@@ -65,11 +69,14 @@ public:
                 bytes -= rounded;
                 blocks--;
                 live[*ptr] = rounded;
+                used += rounded;
                 return Driver::kOk;
             }
             const Status st = driver.alloc(ptr, rounded, stream);
             if (st == Driver::kOk) {
                 live[*ptr] = rounded;
+                used += rounded;
+                if (bytes && !fits(bytes)) give_back(home);
                 return st;
             }
             // out of memory: without the kept blocks, and without the rounding
@@ -97,8 +104,9 @@ public:
             if (it != live.end()) {
                 const size_t size = it->second;
                 live.erase(it);
-                if (stream == home && size <= limit && !driver.capturing(stream)) {
-                    if (bytes + size > limit) give_back(home);
+                used -= size;
+                if (stream == home && fits(size) && !driver.capturing(stream)) {
+                    if (!fits(bytes + size)) give_back(home);
                     kept[size].push_back(ptr);
                     bytes += size;
                     blocks++;
@@ -109,12 +117,12 @@ public:
         return driver.free(ptr, stream);
     }
 
-    // 0: kKeepBytes alone
-    void set_limit(size_t most, Stream home)
+    // 0: none
+    void set_threshold(size_t most, Stream home)
     {
         std::lock_guard<std::mutex> lock(mu);
-        limit = most && most < kKeepBytes ? most : kKeepBytes;
-        if (bytes > limit && !driver.capturing(home)) give_back(home);
+        threshold = most ? most : SIZE_MAX;
+        if (bytes && !fits(bytes) && !driver.capturing(home)) give_back(home);
     }
 
     void usage(size_t *kept_bytes, size_t *kept_count)
@@ -125,6 +133,9 @@ public:
     }
 
 private:
+    // so many kept bytes, beside the blocks in use
+    bool fits(size_t n) const { return n <= kKeepBytes && used <= threshold && n <= threshold - used; }
+
     // Every kept block back to the driver's pool (the caller holds the lock
     // and the home stream is not being captured).
     void give_back(Stream home)
@@ -139,7 +150,7 @@ private:
     std::mutex mu;
     std::unordered_map<void *, size_t> live;               // rounded size of blocks handed out
     std::unordered_map<size_t, std::vector<void *>> kept;  // free blocks by rounded size
-    size_t bytes = 0, blocks = 0, limit = kKeepBytes;
+    size_t used = 0, bytes = 0, blocks = 0, threshold = SIZE_MAX;
 };
 
 }  // namespace pt

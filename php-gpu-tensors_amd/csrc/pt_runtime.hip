@@ -505,7 +505,7 @@ pt_status pt_mem_init(size_t pool_bytes)
 {
     PT_TRY(ensure_init());
     uint64_t threshold = pool_bytes ? (uint64_t)pool_bytes : UINT64_MAX;
-    kept_blocks().set_limit(pool_bytes, g_stream);
+    kept_blocks().set_threshold(pool_bytes, g_stream);
     return check_hip(hipMemPoolSetAttribute(g_pool, hipMemPoolAttrReleaseThreshold, &threshold),
                      "hipMemPoolSetAttribute");
 }

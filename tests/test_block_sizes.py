@@ -130,27 +130,47 @@ int main()
         assert(get(k, MiB));
         is(k, MiB, 1);
     }
-    {  // the limit
+    {  // what is kept, and the threshold on it and the blocks in use together
         Card c;
         Blocks k(Driver{&c});
-        k.set_limit(4 * MiB, 0);
+        put(k, get(k, 5 * MiB));
+        put(k, get(k, Blocks::kKeepBytes));
+        is(k, Blocks::kKeepBytes, 1);
+        put(k, get(k, Blocks::kKeepBytes + 1));
+        is(k, Blocks::kKeepBytes, 1);
+        k.set_threshold(6 * MiB, 0);
+        is(k, 0, 0);
         void *p[6];
         for (auto &b : p) b = get(k, MiB);
         for (int i = 0; i < 6; i++) {
             put(k, p[i]);
-            is(k, (i % 4 + 1) * MiB, i % 4 + 1);
+            is(k, (i + 1) * MiB, i + 1);
         }
+        void *two = get(k, 2 * MiB);  // 8 MiB with those kept
+        is(k, 0, 0);
         assert(c.used == 2 * MiB);
-        put(k, get(k, 5 * MiB));
+        for (int i = 0; i < 5; i++) p[i] = get(k, MiB);  // 7 MiB in use
+        put(k, p[0]);  // 6 with it
+        is(k, 0, 0);
+        put(k, p[1]);
+        put(k, p[2]);
         is(k, 2 * MiB, 2);
-        k.set_limit(MiB, 0);
+        assert(c.used == 6 * MiB);
+        void *big = get(k, 7 * MiB);
+        is(k, 0, 0);
+        put(k, p[3]);
+        is(k, 0, 0);
+        put(k, big);
+        is(k, 0, 0);
+        put(k, two);
+        put(k, p[4]);
+        is(k, 3 * MiB, 2);
+        k.set_threshold(2 * MiB, 0);
         is(k, 0, 0);
         assert(c.used == 0);
-        k.set_limit(0, 0);
+        k.set_threshold(0, 0);
         put(k, get(k, 5 * MiB));
         is(k, 5 * MiB, 1);
-        put(k, get(k, Blocks::kKeepBytes));
-        is(k, Blocks::kKeepBytes, 1);
     }
     for (int s = 0; s < 2; s++) {  // out of memory: what is kept makes room, once, and then the call fails
         Card c;

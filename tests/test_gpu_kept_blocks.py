@@ -106,27 +106,27 @@ def test_other_streams_and_captures_pass_by(lib):
 
 
 def test_bound(lib):
-    """Blocks beyond the bound go back to the driver's pool, and the bound can be lowered."""
-    A.check(lib.pt_mem_init(1 << 20))
-    assert _kept(lib)[0] <= 1 << 20
+    """Blocks in use and kept together stay within the threshold, or none are
+    kept, and the threshold can be lowered."""
+    A.check(lib.pt_mem_init(1))
+    assert _kept(lib) == (0, 0)
+    A.check(lib.pt_free(_alloc(lib, 300_000), None))
+    assert _kept(lib) == (0, 0)
+    A.check(lib.pt_mem_init(1 << 34))
     blocks = [_alloc(lib, 300_000) for _ in range(8)]
     assert len(set(blocks)) == 8
-    for b in blocks:
+    for i, b in enumerate(blocks):
         A.check(lib.pt_free(b, None))
-        assert 0 < _kept(lib)[0] <= 1 << 20
-    before = _kept(lib)
-    big = _alloc(lib, 8 << 20)  # larger than the bound: not kept
-    A.check(lib.pt_free(big, None))
-    assert _kept(lib) == before
+        assert _kept(lib) == ((i + 1) * 327680, i + 1)
     again = [_alloc(lib, 300_000) for _ in range(8)]
-    assert len(set(again)) == 8 and _kept(lib) == (before[0] - before[1] * 327680, 0)
-    for b in again[:2]:
+    assert set(again) == set(blocks) and _kept(lib) == (0, 0)
+    for b in again[:4]:
         A.check(lib.pt_free(b, None))
-    assert _kept(lib) == (2 * 327680, 2)
-    A.check(lib.pt_mem_init(400_000))
+    A.check(lib.pt_mem_init(3 * 327680))  # with the four in use
     assert _kept(lib) == (0, 0)
-    for b in again[2:]:
+    for b in again[4:]:
         A.check(lib.pt_free(b, None))
+        assert _kept(lib)[0] <= 3 * 327680
     A.check(lib.pt_mem_init(0))
 
 
