@@ -2111,8 +2111,8 @@ static int row_waves()
 }
 
 // Rows whose length, pitch and base are multiples of 16 bytes are read in
-// aligned 16-byte chunks; ragged rows (RAG) too, from their first 16-byte
-// boundary on.  (Chunks from the row's first element, across lines, were
+// aligned 16-byte chunks; ragged rows (RAG) too, from their first 128-byte
+// line on.  (Chunks from the row's first element, across lines, were
 // slower than 4-byte loads: sum, max, argMax and var of [8192, 4095] fp32
 // 126 us with nontemporal loads and 117 us with cached ones, against 112.)
 // Ragged rows of at most 256 elements keep 4-byte (2-byte) loads except for

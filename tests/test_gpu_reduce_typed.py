@@ -24,7 +24,7 @@ def G():
 
 
 def _ints(shape, dt, seed):
-    """Small whole numbers (every sum exact, many ties) with a NaN and both infinities in some columns."""
+    """Small whole numbers: every sum exact, many ties."""
     from phptensors import synthetic
     x = np.round(synthetic.uniform(shape, -40.0, 40.0, seed=seed)).astype(np.float32)
     return x, O.to_storage(x.astype(np.float64) if dt == O.F64 else x, dt)
@@ -95,6 +95,27 @@ def test_nonfinite_values(G, dt, axis):
         assert np.isnan(got[0])
     else:
         assert np.all(np.isnan(got[:8])) and np.all(np.isfinite(got[8:]))
+
+
+@pytest.mark.parametrize("dt", DTS, ids=NAMES.get)
+@pytest.mark.parametrize("shape", [(5003, 301), (9001, 1003)], ids=str)
+def test_nonfinite_values_of_a_straddling_lane(G, dt, shape):
+    """The same in the last columns, which the lane that straddles the row's
+    end loads one by one, in the first, a middle and the last of several row
+    slices."""
+    x, _ = _ints(shape, dt, 6)
+    last, mid = shape[0] - 1, shape[0] // 2
+    x[mid, -1] = x[0, -2] = x[last, -3] = np.nan
+    x[:, -4], x[:, -5], x[:, -6] = -np.inf, np.inf, np.nan
+    x[last, -7], x[0, -8] = np.inf, -np.inf
+    x[:, -9], x[mid, -9] = -np.inf, 3.0
+    xs = O.to_storage(x.astype(np.float64) if dt == O.F64 else x, dt)
+    for op in ("argmax", "argmin"):
+        assert np.array_equal(G.arg_reduce(xs, dt, op, 0), O.arg_reduce(xs, dt, op, 0)), op
+    for op in ("sum", "max", "min"):
+        assert np.array_equal(G.reduce(xs, dt, op, 0)[0], O.reduce(xs, dt, op, 0)[0], equal_nan=True), op
+    got = np.asarray(G.moments(xs, dt, 0)).ravel()
+    assert np.all(np.isnan(got[-9:])) and np.all(np.isfinite(got[:-9]))
 
 
 def test_variance_far_from_zero(G):
