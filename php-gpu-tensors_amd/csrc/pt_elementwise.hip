@@ -478,7 +478,7 @@ __global__ __launch_bounds__(256) void k_where_vec(Opnd cond, Opnd x, Opnd y, vo
 
 // Casts between the 32- and 16-bit floating types; V elements are 16 bytes
 // of the wider type.
-template <int DTI, int DTO, bool NT>
+template <int DTI, int DTO>
 __global__ __launch_bounds__(256) void k_cast_vec(Opnd x, void *__restrict__ out, size_t total, unsigned cols)
 {
     using TI = typename VecT<DTI>::T;
@@ -488,10 +488,10 @@ __global__ __launch_bounds__(256) void k_cast_vec(Opnd x, void *__restrict__ out
     if (!q.valid) return;
     TI t[V];
     TO z[V];
-    fetch<OPND_ANY, TI, V, NT>(x, q, cols, t);
+    fetch<OPND_ANY, TI, V, false>(x, q, cols, t);
 #pragma unroll
     for (int k = 0; k < V; k++) z[k] = VecT<DTO>::from(VecT<DTI>::to(t[k]));
-    put<TO, V, NT>((TO *)out, q, z);
+    put<TO, V, false>((TO *)out, q, z);
 }
 
 // ------------------------------------------------------------------ unary
@@ -717,24 +717,30 @@ static unsigned opnd_cols(const EwShape &s)
 }
 
 // Streaming accesses bypass cache retention (nontemporal) in calls through
-// aligned chunks that move `least` bytes or more.  Ordinarily a gigabyte: the
-// 256 MB Infinity Cache then holds nothing that the next call could read.  A
-// chain of eager calls (add, gt, where, multiply, add, astype; cached against
-// nontemporal): [8000, 3001] bf16 150 against 166 us, [8000, 3000] fp32 201
-// against 215, [16000, 8001] fp32 (1.5 GB a call) 1050 against 992, and tanh
-// of [16384, 8192] fp32 (1.07 GB) 175 against 165.
-// Calls on two full operands stream from 256 MB on: with the output they are
-// three streams that do not fit the cache together, and what they evict is
-// the result of the call before.  x + m of [8192, 4096] fp32 (403 MB) 69.4
-// cached and 62.6 us nontemporal, y * x, + m and tanh of it 150 and 137, of
-// [8192, 8192] 314 and 285, of [16000, 8000] bf16 328 and 302; the six calls
-// of [4096, 4096] fp32 (201 MB a sum) 147 and 150.
-constexpr size_t kStreamBytes = 1000000000, kStreamPairBytes = (size_t)256 << 20;
-static bool streams(size_t bytes, size_t least, std::initializer_list<const void *> ptrs)
+// aligned chunks whose tensors do not fit the 256 MB Infinity Cache together:
+// there is nothing left in it for the next call, and what such a call evicts is
+// the result of the call before.  The line lies at 272 MB of one full operand
+// and the output, at 344 MB of more operands.  Eager calls on one of four
+// inputs in turn, us cached against nontemporal, by size of a tensor:
+//   fp32 x * 2       128 MB 40.4 / 42.9, 144 MB 51.6 / 47.7, 256 MB 89.7 / 84.0
+//   fp32 tanh        128 MB 41.0 / 42.0, 144 MB 51.3 / 46.7, 512 MB 173 / 163
+//   fp32 x + m       100 MB 42.8 / 44.7, 112 MB 49.9 / 50.1, 120 MB 56.0 / 53.2,
+//                    192 MB 96.2 / 86.4, 512 MB 251 / 233
+//   fp32 where       100 MB 44.8 / 47.5, 120 MB 58.1 / 56.2, 192 MB 97.9 / 90.4
+//   bf16 x * 2       128 MB 41.5 / 43.5, 144 MB 51.8 / 48.7
+//   bf16 x + m       112 MB 52.1 / 53.2, 120 MB 57.7 / 56.3, 192 MB 94.8 / 90.0
+// and chains of them alike (bias, scale and tanh of fp32 128 MB 160 / 178, 192 MB
+// 273 / 262).  Calls that are as fast or faster cached at every size are not
+// asked: 16-bit unary calls (512 MB 171 / 179), 16-bit where (272 / 294), 16-bit
+// operands with one row or one value per row (184 / 188), and calls whose
+// chunks have 32 bytes on one side, two stores of a lane to every line (a cast
+// from bf16 to fp32: 128 MB 71 / 99, 512 MB 272 / 402).
+constexpr size_t kStreamOne = (size_t)272 << 20, kStreamMore = (size_t)344 << 20;
+static bool streams(size_t bytes, int operands, std::initializer_list<const void *> ptrs)
 {
     for (const void *p : ptrs)
         if ((uintptr_t)p & 15) return false;
-    return bytes >= least;
+    return bytes >= (operands > 1 ? kStreamMore : kStreamOne);
 }
 
 static bool vec_float(int dt) { return dt == PT_FLOAT32 || dt == PT_FLOAT16 || dt == PT_BFLOAT16; }
@@ -779,17 +785,23 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
     if (vec) {
         if (reverse) std::swap(oa, ob);
         const size_t total = (size_t)s.total;
-        const bool pair = oa.mode == OPND_FLAT && ob.mode == OPND_FLAT;
-        const bool nt = streams(total * (dtype_size(dta) * (scalar ? 1 : 2) + dtype_size(dto)),
-                                pair ? kStreamPairBytes : kStreamBytes,
+        auto full = [](const Opnd &o) { return o.mode == OPND_FLAT || o.mode == OPND_IMM; };
+        const int operands = (oa.mode == OPND_FLAT) + (ob.mode == OPND_FLAT);
+        const bool nt = dto == dta && (dta == PT_FLOAT32 || (full(oa) && full(ob))) &&
+                        streams(total * dtype_size(dta) * (size_t)(operands + 1), operands,
                                 {oa.mode == OPND_FLAT ? oa.p : nullptr, ob.mode == OPND_FLAT ? ob.p : nullptr, out});
         with_vec_dtype(dta, [&](auto D) {
             constexpr int DT = decltype(D)::value;
             const unsigned grid = grid_for(s.total, 16 / (int)sizeof(typename VecT<DT>::T)), cols = opnd_cols(s);
             auto go = [&](auto O, auto MA, auto MB) {
                 constexpr int DO = decltype(O)::value, A = decltype(MA)::value, B = decltype(MB)::value;
-                if (nt) k_binary_vec<DT, DO, true, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
-                else k_binary_vec<DT, DO, false, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
+                if constexpr (DO == DT) {
+                    if (nt) {
+                        k_binary_vec<DT, DO, true, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
+                        return;
+                    }
+                }
+                k_binary_vec<DT, DO, false, A, B><<<grid, 256, 0, st_>>>(oa, ob, out, op, total, cols);
             };
             // the layouts of most calls have kernels of their own: y * z of
             // a row and [16384, 8192] fp32 took 181 us with the layouts read
@@ -802,7 +814,7 @@ static pt_status binary_impl(const void *a, int dta, const size_t *sa, size_t of
             using CL = std::integral_constant<int, OPND_COL>;
             using AN = std::integral_constant<int, OPND_ANY>;
             if (dto != dta) go(std::integral_constant<int, PT_FLOAT32>{}, AN{}, AN{});
-            else if (pair) go(D, FL{}, FL{});
+            else if (oa.mode == OPND_FLAT && ob.mode == OPND_FLAT) go(D, FL{}, FL{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_IMM) go(D, FL{}, IM{});
             else if (oa.mode == OPND_FLAT && ob.mode == OPND_ROWS) go(D, FL{}, RW{});
             else if (oa.mode == OPND_ROWS && ob.mode == OPND_FLAT) go(D, RW{}, FL{});
@@ -872,7 +884,8 @@ pt_status pt_unary(const void *input, int dtype, const size_t *strides, size_t o
     Opnd ox;
     if (vec_float(dtype) && as_opnd(s, s.sa, px, ox)) {
         const size_t total = (size_t)s.total;
-        const bool nt = streams(total * dtype_size(dtype) * 2, kStreamBytes, {ox.mode == OPND_FLAT ? px : nullptr, out});
+        const bool nt = dtype == PT_FLOAT32 &&
+                        streams(total * dtype_size(dtype) * 2, 1, {ox.mode == OPND_FLAT ? px : nullptr, out});
         with_vec_dtype(dtype, [&](auto D) {
             constexpr int DT = decltype(D)::value;
             const unsigned grid = grid_for(s.total, 16 / (int)sizeof(typename VecT<DT>::T)), cols = opnd_cols(s);
@@ -889,8 +902,10 @@ pt_status pt_unary(const void *input, int dtype, const size_t *strides, size_t o
                 else if (op == PT_OP_EXP) go(std::integral_constant<int, PT_OP_EXP>{}, N);
                 else go(std::integral_constant<int, -1>{}, N);
             };
-            if (nt) pick(std::true_type{});
-            else pick(std::false_type{});
+            if constexpr (DT == PT_FLOAT32) {
+                if (nt) return pick(std::true_type{});
+            }
+            pick(std::false_type{});
         });
     } else {
         EwShape32 s32;
@@ -934,15 +949,12 @@ pt_status pt_cast(const void *input, int dtype_in, const size_t *strides, size_t
     EwShape32 s32;
     if (vec_float(dtype_in) && vec_float(dtype_out) && dtype_in != dtype_out && as_opnd(s, s.sa, px, ox)) {
         const size_t total = (size_t)s.total;
-        const bool nt = streams(total * (dtype_size(dtype_in) + dtype_size(dtype_out)), kStreamBytes,
-                                {ox.mode == OPND_FLAT ? px : nullptr, out});
         with_vec_dtype(dtype_in, [&](auto I) {
             with_vec_dtype(dtype_out, [&](auto O) {
                 constexpr int DI = decltype(I)::value, DO = decltype(O)::value;
                 if constexpr (DI != DO) {
                     const unsigned grid = grid_for(s.total, 8);
-                    if (nt) k_cast_vec<DI, DO, true><<<grid, 256, 0, st_>>>(ox, out, total, opnd_cols(s));
-                    else k_cast_vec<DI, DO, false><<<grid, 256, 0, st_>>>(ox, out, total, opnd_cols(s));
+                    k_cast_vec<DI, DO><<<grid, 256, 0, st_>>>(ox, out, total, opnd_cols(s));
                 }
             });
         });
@@ -973,17 +985,19 @@ pt_status pt_where(const void *cond, int dtype_cond, const size_t *strides_cond,
         const size_t total = (size_t)s.total;
         // a floating condition holds unless it is +0 or -0; integers and bool unless they are 0
         const uint32_t mask = dtype_is_floating(dtype_cond) ? (csz == 4 ? 0x7fffffffu : 0x7fffu) : 0xffffffffu;
-        const bool nt = streams(total * (size_t)(csz + 3 * esz), kStreamBytes,
-                                {oc.mode == OPND_FLAT ? cond : nullptr, ox.mode == OPND_FLAT ? x : nullptr,
-                                 oy.mode == OPND_FLAT ? y : nullptr, out});
+        const bool fc = oc.mode == OPND_FLAT, fx = ox.mode == OPND_FLAT, fy = oy.mode == OPND_FLAT;
+        const bool nt = esz == 4 && streams(total * (size_t)(csz * fc + esz * (fx + fy + 1)), fc + fx + fy,
+                                            {fc ? cond : nullptr, fx ? x : nullptr, fy ? y : nullptr, out});
         auto go = [&](auto E, auto C, auto N) {
             constexpr int ES = decltype(E)::value, CS = decltype(C)::value;
             k_where_vec<ES, CS, decltype(N)::value><<<grid_for(s.total, 16 / ES), 256, 0, st_>>>(oc, ox, oy, out, mask,
                                                                                               total, opnd_cols(s));
         };
         auto pick = [&](auto E, auto C) {
-            if (nt) go(E, C, std::true_type{});
-            else go(E, C, std::false_type{});
+            if constexpr (decltype(E)::value == 4) {
+                if (nt) return go(E, C, std::true_type{});
+            }
+            go(E, C, std::false_type{});
         };
         auto by_cond = [&](auto E) {
             if (csz == 1) pick(E, std::integral_constant<int, 1>{});

@@ -134,3 +134,25 @@ def test_three_dimensions_and_empty(dt):
     _same(_up(xs, dt) + _up(bs, dt), x + b, dt)
     e = _up(xs[:0], dt)
     assert (e + 1.0).getShape() == [0, 5, 9] and e.tanh().getShape() == [0, 5, 9]
+
+
+@pytest.mark.parametrize("dt", list(NAMES), ids=NAMES.get)
+def test_calls_past_the_caches(dt):
+    """Tensors of 290 MB, an odd number of elements: the nontemporal forms give
+    the bits of the cached ones (which short rows of the same values run)."""
+    from phptensors import CudaArray
+    rows, cols = (18311, 4097) if dt == O.F32 else (36601, 4099)
+    _, a = _values((1, cols), dt, 10)
+    _, b = _values((1, cols), dt, 11)
+    tall = lambda s: _up(np.repeat(s, rows, 0), dt)
+    x, m, x1, m1 = tall(a), tall(b), _up(a, dt), _up(b, dt)
+    c, c1 = CudaArray.full([rows, 1], 1.25, NAMES[dt]), CudaArray.full([1, 1], 1.25, NAMES[dt])
+    for name, big, small in (("pair", x + m, x1 + m1), ("scalar", x * 0.5, x1 * 0.5), ("reverse", 0.5 - x, 0.5 - x1),
+                             ("row", x - m1, x1 - m1), ("row first", m1 - x, m1 - x1), ("column", x * c, x1 * c1),
+                             ("column first", c - x, c1 - x1), ("unary", x.neg(), x1.neg()), ("quotient", x / m, x1 / m1),
+                             ("tanh", x.tanh(), x1.tanh()), ("where", CudaArray.where(x.gt(0), x, m),
+                                                              CudaArray.where(x1.gt(0), x1, m1))):
+        got, ref = big.toBits(), small.toBits()
+        assert got.shape == (rows, cols) and got.dtype == ref.dtype, name
+        assert np.array_equal(got.view(np.uint8), np.broadcast_to(ref, (rows, cols)).copy().view(np.uint8)), name
+        del big, got
