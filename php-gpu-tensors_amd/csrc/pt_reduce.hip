@@ -1753,8 +1753,8 @@ __device__ __forceinline__ void fold_store(void *out, int out_dt, size_t i, type
 // columns in registers, and meet in LDS in wave order.  With one slice per
 // column the block writes the result; otherwise it writes a partial per
 // slice and k_col_final_t merges them in slice order.  Rows need no
-// alignment; the lane that straddles the last column loads its columns one
-// by one.
+// alignment; the lane that straddles the last column loads the row's last V
+// columns and keeps its own.
 // Bound by HBM: [20000, 784] fp32 is 62.7 MB.  Argmax and variance took
 // 153 us each on the generic kernels (a 120-byte state of every dtype, one
 // element per lane and load); sum, max, argmax and variance of it one after
@@ -1774,11 +1774,13 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
     const size_t split = blockIdx.y, o = blockIdx.z;
     const size_t lo = split * slice;
     const size_t hi = lo + slice < n ? lo + slice : n;
-    const int valid = col >= inner ? 0 : inner - col < (size_t)V ? (int)(inner - col) : V;
+    // (the host gives V > 1 only rows of V columns or more)
+    const size_t at = col + V <= inner ? col : inner - V;
+    const int skip = col >= inner ? V : (int)(col - at);  // columns of the lane before
     F acc[V];
     size_t taken = 0;  // rows this wave has folded in
-    if (valid == V) {
-        const S *x = (const S *)xin + o * n * inner + col;
+    if (skip < V) {
+        const S *x = (const S *)xin + o * n * inner + at;
         size_t r = lo + wave;
         if (r < hi) taken = (hi - r + 3) / 4;
         if constexpr (OP == R_VAR) {
@@ -1803,22 +1805,6 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
 #pragma unroll
             for (int k = 0; k < V; k++) acc[k].add(v[k], (int)r);
         }
-    } else if (valid) {
-        const S *x = (const S *)xin + o * n * inner + col;
-        size_t r = lo + wave;
-        if (r < hi) taken = (hi - r + 3) / 4;
-#pragma unroll
-        for (int k = 0; k < V; k++)
-            if (k < valid && r < hi) acc[k].begin(RT<DT>::cv(x[r * inner + k]));
-        if constexpr (OP == R_VAR && sizeof(C) == 8) {
-            static_assert(V <= 2, "one column is left of a float64 pack");
-            for (; r + 12 < hi; r += 16)
-                acc[0].add4(x[r * inner], x[(r + 4) * inner], x[(r + 8) * inner], x[(r + 12) * inner]);
-        }
-        for (; r < hi; r += 4)
-#pragma unroll
-            for (int k = 0; k < V; k++)
-                if (k < valid) acc[k].add(RT<DT>::cv(x[r * inner + k]), (int)r);
     }
     __shared__ LdsSlot<P> part[3][64 * V];
     if (wave > 0)
@@ -1831,7 +1817,7 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
     if (wave != 0) return;
 #pragma unroll
     for (int k = 0; k < V; k++) {
-        if (k >= valid) continue;
+        if (k < skip) continue;
         P a = acc[k].part(taken);
 #pragma unroll
         for (int w = 0; w < 3; w++) {
@@ -1839,8 +1825,8 @@ __global__ __launch_bounds__(256) void k_col_reduce_t(const void *__restrict__ x
             memcpy(&b, part[w][k * 64 + lane].raw, sizeof(P));
             a = F::merge(a, b);
         }
-        if (partial) partial[(o * gridDim.y + split) * inner + col + k] = a;
-        else fold_store<C, OP>(out, out_dt, o * inner + col + k, a, n, correction, take_sqrt);
+        if (partial) partial[(o * gridDim.y + split) * inner + at + k] = a;
+        else fold_store<C, OP>(out, out_dt, o * inner + at + k, a, n, correction, take_sqrt);
     }
 }
 
@@ -2117,7 +2103,13 @@ static int row_waves()
 // 126 us with nontemporal loads and 117 us with cached ones, against 112.)
 // Ragged rows of at most 256 elements keep 4-byte (2-byte) loads except for
 // variances: one chunk a lane at most, and the fusion executor's row chains
-// restate their order of additions.
+// restate their order of additions (ragged_by_element: and some longer ones).
+// Ragged rows of 5 to 16 chunks take a wave each as soon as that gives every
+// SIMD one: with a block per row most of its waves hold one partial chunk or
+// none, for the price of the exchange between them.  sum / argMax / var, us, of
+// [39024, 1025] fp32 50 / 74 / 82 with 8 waves a row, 27 / 27 / 27 with one; [19521,
+// 2049] 31 / 41 / 45 and 24 / 25 / 25; [13328, 3001] 28 / 29 / 30 and 25 / 25 / 26;
+// var of [31234, 2049] bf16 43 and 27, of [38986, 513] fp64 61 and 41.
 template <int DT, int OP, bool RAG>
 static void launch_rows_wide(const void *x, size_t rows, int n, size_t ld, void *out, int out_dt,
                              int correction, int take_sqrt, hipStream_t s)
@@ -2127,6 +2119,10 @@ static void launch_rows_wide(const void *x, size_t rows, int n, size_t ld, void 
     const int chunks = (int)(((long long)n + 64 * V - 1) / (64 * V));
     dim3 grid1((unsigned)rows), grid4((unsigned)((rows + 3) / 4));
     const double rn = 1.0 / (double)n, rc = 1.0 / (double)(n - correction);
+    if (RAG && chunks > 4 && chunks <= 16 && rows >= 1024) {
+        k_row_reduce<DT, OP, V, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt, rn, rc);
+        return;
+    }
     if constexpr (DT == PT_FLOAT32) {
         if (row_waves() == 8 && chunks > 4 && chunks <= 16) {
             dim3 block8(512);
@@ -2172,6 +2168,21 @@ static void launch_rows_wide(const void *x, size_t rows, int n, size_t ld, void 
         k_row_reduce<DT, OP, V, 1, RAG><<<grid4, block, 0, s>>>(x, rows, n, ld, out, out_dt, correction, take_sqrt, rn, rc);
 }
 
+// Ragged rows that the element loads read faster: variances never, others of
+// up to 256 elements always, and those whose 16-byte chunks fill too little of
+// a wave-wide one.  us by element against 16 bytes a lane: sum of [249027, 257]
+// bf16 38 / 52, [212624, 301] 32 / 42, [166233, 385] 37 / 34; argMax of [212624, 301]
+// bf16 43 / 61, [83224, 769] 28 / 34, [63936, 1001] 29 / 27; argMax of [106312, 301]
+// fp32 25 / 28, [83116, 385] 29 / 24.
+template <int DT, int OP>
+static bool ragged_by_element(int n)
+{
+    constexpr bool ARG = OP == R_ARGMAX || OP == R_ARGMIN;
+    if constexpr (OP == R_VAR) return false;
+    else if constexpr (sizeof(typename RT<DT>::S) == 2) return n <= (ARG ? 800 : 352);
+    else return n <= (ARG && DT == PT_FLOAT32 ? 320 : 256);
+}
+
 template <int DT, int OP>
 static void launch_rows_t(const void *x, size_t rows, int n, size_t ld, void *out, int out_dt,
                           int correction, int take_sqrt, hipStream_t s)
@@ -2179,7 +2190,7 @@ static void launch_rows_t(const void *x, size_t rows, int n, size_t ld, void *ou
     constexpr int V = RT<DT>::V;
     if (n % V == 0 && ld % V == 0 && aligned16(x))
         launch_rows_wide<DT, OP, false>(x, rows, n, ld, out, out_dt, correction, take_sqrt, s);
-    else if ((OP == R_VAR || n > 256) && n < 0x7fff0000)  // (the wide kernels count elements past the row's end in an int)
+    else if (!ragged_by_element<DT, OP>(n) && n < 0x7fff0000)  // (the wide kernels count elements past the row's end in an int)
         launch_rows_wide<DT, OP, true>(x, rows, n, ld, out, out_dt, correction, take_sqrt, s);
     else
         k_row_reduce<DT, OP, 1, 1><<<dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s>>>(
@@ -2236,9 +2247,13 @@ static int result_dtype(int dtype, int rop)
 // slices that 64-column blocks ask for, and so their order of additions;
 // maxima and minima take more only while their scratch stays within the
 // no-allocation entry's megabyte, which then holds it for the same calls as
-// ever.  Where 16-byte packs leave sums fewer than two blocks a CU they are
-// read in narrower ones.  sum, max, argMax and var of [8000, 3001] bf16
-// along axis 0: 138 us with nontemporal loads and 264 blocks a call, 102 us.
+// ever.  Where unaligned 16-byte packs leave fewer than two blocks a CU they
+// are read in narrower ones, as are 16-bit variances (eight states in double a
+// lane) and variances over few rows.  us with 16 bytes a lane against narrower:
+// max of [249027, 257] bf16 63 / 55, argMax 117 / 66, var 197 / 73; var of [21326,
+// 3001] bf16 64 / 53, of [124513, 257] fp32 61 / 47, of [61, 65537] bf16 13 / 6.
+// (With the straddling lane's columns loaded one by one: sum, max of [124513,
+// 257] bf16 86 and 112, of [7806, 4099] fp32 47 and 41, now 30 and 29.)
 template <int DT, int OP>
 static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inner, void *out, int out_dt,
                                int correction, int take_sqrt, hipStream_t s)
@@ -2269,7 +2284,9 @@ static pt_status launch_cols_t(const void *x, size_t outer, size_t n, size_t inn
     splits = (n + slice - 1) / slice;
     P *partial = nullptr;
     if (splits > 1) PT_TRY(scratch_alloc((void **)&partial, sizeof(P) * outer * splits * inner, s));
-    const int width = !vec ? 1 : packed || !ORDERED || vec_blocks * splits * outer >= 512 ? V : W;
+    constexpr bool VAR16 = OP == R_VAR && sizeof(typename RT<DT>::S) == 2;
+    const bool wide = vec_blocks * splits * outer >= 512;
+    const int width = !vec ? 1 : packed ? (OP == R_VAR && splits == 1 && !wide ? W : V) : wide && !VAR16 ? V : W;
     auto go = [&](auto N, auto T) {
         constexpr int C = decltype(N)::value;
         const dim3 grid((unsigned)((inner + 64 * C - 1) / (64 * C)), (unsigned)splits, (unsigned)outer);
