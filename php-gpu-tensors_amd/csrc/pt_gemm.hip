@@ -157,7 +157,7 @@ struct TileLoader {
     __device__ __forceinline__ void load(const S *base, long long s_r, long long s_k, int r0,
                                          int r_total, int k0, int K, int tid, int vec = 0)
     {
-        const bool moves = EDGE && r0 + R > r_total;  // a load may straddle r_total (uniform)
+        const bool moves = EDGE && r0 + R > r_total && r_total % RL != 0;  // a load may straddle r_total (uniform)
         if constexpr (KM) {
             // pack p: k row p / (R / PK), r pack p % (R / PK); a wave reads
             // whole rows of r
@@ -1259,10 +1259,18 @@ pt_status pt_matmul(const void *a, const void *b, void *c, int dtype,
     if (dtype == PT_FLOAT32 && g_tile_override < 0 && !tuned && (tile == TILE_256x256 || tile == TILE_128x128_W8)) {
         GemmArgs whole = g;
         whole.ksplit = 1;
-        // (a K of no multiple of 16 only where neither kernel splits it: both
-        // then add in the same order)
+        // A K of no multiple of 16 only where neither kernel splits it (both
+        // then add in the same order) and K is long enough to pay for the
+        // ring's tail form, which fills four stages before its first MFMA, one
+        // workgroup a CU.  Ring against 8 waves, us (each layout's best and
+        // worst): 4000 x 1024 (256 tiles) K 100 15.1/14.7 to 16.2/14.9, K 200
+        // 20.5/21.5 to 21.5/21.1, K 500 37/44; 8 x 776 x 2048 (896 tiles) K 20
+        // 29/22, K 100 50/41 to 54/42, K 260 85/82 to 89/80, K 500 135/144 to
+        // 137.5/136.8, K 1000 250/272; 4096 x 4096 K 260 86/82 to 90/81, K 500
+        // 136/142 to 141/138.
         const long long t128 = ((g.M + 127) / 128) * (long long)((g.N + 127) / 128) * batch;
-        if (gemm_f32r_eligible(whole, a_kc, b_kc) && (g.K % 16 == 0 || g.K < 128 || t128 >= 256)) tile = TILE_F32_RING;
+        const bool tail = t128 >= 256 && g.K >= (t128 == 256 ? 200 : 384);
+        if (gemm_f32r_eligible(whole, a_kc, b_kc) && (g.K % 16 == 0 || tail)) tile = TILE_F32_RING;
     }
     int bm = kTiles[tile].bm, bn = kTiles[tile].bn;
     const int BK = (dtype == PT_FLOAT32 ? 16 : 32) * kTiles[tile].kmul;

@@ -43,7 +43,7 @@ def _check(dt, bmnk, ta, tb, wide):
 @pytest.mark.parametrize("tb", [False, True], ids=["B", "Bt"])
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 12, 20, 31, 33, 36, 100, 127, 1000, 1004])
 def test_fp32_k_tails(ta, tb, k):
-    """The ring kernel's last step at every kind of remainder, whole and split K."""
+    """The last K step at every kind of remainder, whole and split K."""
     for b, m, n in ((1, 128, 128), (2, 260, 132), (1, 256, 384)):
         _check(O.F32, (b, m, n, k), ta, tb, 0)
     _check(O.F32, (1, 128, 132, 4 * k + 2048), ta, tb, 0)
@@ -79,13 +79,18 @@ def test_fp32_ring_beside_nan(ta, tb, before, k):
         x, xm, xo, xp = _padded((m, k), ta, before, m + k)
         y, ym, yo, yp = _padded((k, n), tb, before, n + k)
         da, db, dc = A.to_device(xm), A.to_device(ym), A.DeviceBuffer(4 * m * n)
-        A.matmul(da.ptr + 4 * xo, db.ptr + 4 * yo, dc.ptr, A.FLOAT32, (m, k), [1, xp] if ta else [xp, 1],
-                 (k, n), [1, yp] if tb else [yp, 1], (m, n))
-        assert A.backend_info().last_matmul.decode() == "mfma-fp32-ring"
-        assert np.array_equal(dc.download(np.float32, (m, n)), (x.astype(np.float64) @ y.astype(np.float64)))
+        for tile in (38, -1):  # the ring, and what the dispatch takes for so short a K
+            A.check(lib.pt_matmul_set_tile(tile))
+            try:
+                A.matmul(da.ptr + 4 * xo, db.ptr + 4 * yo, dc.ptr, A.FLOAT32, (m, k), [1, xp] if ta else [xp, 1],
+                         (k, n), [1, yp] if tb else [yp, 1], (m, n))
+            finally:
+                lib.pt_matmul_set_tile(-1)
+            assert (A.backend_info().last_matmul.decode() == "mfma-fp32-ring") == (tile == 38)
+            assert np.array_equal(dc.download(np.float32, (m, n)), (x.astype(np.float64) @ y.astype(np.float64)))
 
 
-@pytest.mark.parametrize("k", [777, 1002])
+@pytest.mark.parametrize("k", [383, 385, 777, 1002])
 def test_fp32_ring_beside_nan_on_a_full_grid(k):
     """The same where the tiles alone fill the CUs, as columns of wider tensors."""
     from phptensors import CudaArray, _abi, synthetic
@@ -98,7 +103,7 @@ def test_fp32_ring_beside_nan_on_a_full_grid(k):
         w[:, 4:4 + k] = v
         wide.append(CudaArray.fromNumpy(w).slice(":", [4, 4 + k]))
     got = wide[0].matmul(wide[1].T).toNumpy()
-    assert _abi.backend_info().last_matmul.decode() == "mfma-fp32-ring"
+    assert (_abi.backend_info().last_matmul.decode() == "mfma-fp32-ring") == (k >= 384)
     assert np.array_equal(got, x.astype(np.float64) @ y.astype(np.float64).T)
 
 
