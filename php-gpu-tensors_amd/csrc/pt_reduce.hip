@@ -2510,6 +2510,16 @@ static pt_status reduce_driver(const void *input, void *output, int dtype, int r
 // Rows may start anywhere and have any length: [6000, 1001] bf16 softmax
 // 20.0 -> 10.8 us and layerNorm 21.2 -> 11.7 us against the streaming
 // kernels that rows of no whole chunks ran before.
+// Ragged fp32 rows of 5 to 8 chunks take a wave each as soon as that gives
+// every SIMD one (as the reductions' ragged rows).  softmax / layerNorm, us, by
+// streaming, by 8 waves a row and by one: [31219, 1025] 93 / 108, 101 / 87 and 53 /
+// 69, [3902, 1025] 13.2 / 13.3, 16.9 / 16.3 and 11.0 / 12.8, [15632, 2047] 79 / 89, 55 /
+// 50 and 43 / 42, [1074, 2047] 8.4 / 9.5, 7.4 / 8.4 and 7.5 / 7.6.
+static bool ragged_wave(size_t rows, int chunks, int n, size_t ld, const void *x)
+{
+    return chunks > 4 && chunks <= 8 && rows >= 1024 && (n % 4 != 0 || ld % 4 != 0 || !aligned16(x));
+}
+
 template <int DT, int NCH, int WPR, typename OS>
 static void launch_softmax_nch(const void *x, size_t rows, int n, size_t ld, OS *y, hipStream_t s)
 {
@@ -2526,6 +2536,7 @@ static void launch_softmax_rows(const void *x, size_t rows, int n, size_t ld, OS
     constexpr bool narrow = sizeof(typename RT<DT>::C) == 4;
     const int chunks = (int)(((long long)n + 64 * V - 1) / (64 * V));
     if constexpr (DT == PT_FLOAT32) {
+        if (ragged_wave(rows, chunks, n, ld, x)) return launch_softmax_nch<DT, 8, 1>(x, rows, n, ld, y, s);
         if (chunks > 4 && chunks <= 16 && row_waves() == 8) return launch_softmax_nch<DT, 2, 8>(x, rows, n, ld, y, s);
     }
     switch (chunks) {
@@ -2595,6 +2606,7 @@ static void launch_layernorm_rows(const void *x, size_t rows, int n, CT eps, con
     constexpr int V = RT<DT>::V;
     const int chunks = (int)(((long long)n + 64 * V - 1) / (64 * V));
     if constexpr (DT == PT_FLOAT32 && sizeof(CT) == 4) {
+        if (ragged_wave(rows, chunks, n, n, x)) return launch_layernorm_nch<DT, 8, 1, PDT>(x, rows, n, eps, g, b, y, s);
         if (chunks > 4 && chunks <= 16 && row_waves() == 8)
             return launch_layernorm_nch<DT, 2, 8, PDT>(x, rows, n, eps, g, b, y, s);
     }

@@ -48,10 +48,46 @@ def test_ragged_rows(dt, n):
 
 
 @pytest.mark.parametrize("dt", list(NAMES), ids=NAMES.get)
+@pytest.mark.parametrize("rows", [1023, 1026])
+@pytest.mark.parametrize("n", [321, 353, 801, 1025, 2049, 4095, 4099, 8191])
+def test_ragged_rows_of_a_full_grid(dt, rows, n):
+    """Where the rows alone fill the chip, up to 16 chunks take a wave each; a
+    block of four of them ends past the last row."""
+    from phptensors import CudaArray, synthetic
+    x = synthetic.normal((rows, n), 0.25, 1.0, seed=n)
+    x[1] = np.round(x[1] * 2) / 2
+    xs = O.to_storage(x.astype(np.float64) if dt == O.F64 else x, dt)
+    a, x = CudaArray.fromNumpy(xs, NAMES[dt]), O.from_storage(xs, dt).astype(np.float64)
+    u = 2.0 ** -53 if dt == O.F64 else 2.0 ** -24  # bounds as above
+    assert np.all(np.abs(a.sum(1).toNumpy().astype(np.float64) - x.sum(1)) <= n * u * np.abs(x).sum(1))
+    assert np.array_equal(a.max(1).toNumpy().astype(np.float64), x.max(1))
+    assert np.array_equal(a.argMax(1).toNumpy(), x.argmax(1))
+    assert np.array_equal(a.argMin(1).toNumpy(), x.argmin(1))
+    assert np.allclose(a.var(1).toNumpy().astype(np.float64), x.var(1), rtol=32 * u * n ** 0.5, atol=0)
+
+
+@pytest.mark.parametrize("dt", list(NAMES), ids=NAMES.get)
 @pytest.mark.parametrize("n", LENGTHS)
 def test_ragged_softmax_and_layernorm(dt, n):
-    from phptensors import CudaArray, synthetic
     x, whole, view = _arrays(dt, n, n + 7)
+    _check_normalized(dt, n, x, (whole, view))
+
+
+@pytest.mark.parametrize("rows", [1023, 1024, 1026])
+@pytest.mark.parametrize("n", [1025, 1281, 1534, 2047])
+def test_ragged_normalization_of_a_full_grid(rows, n):
+    """fp32 rows that take a wave each, and those one row short of it."""
+    from phptensors import CudaArray, synthetic
+    x = synthetic.normal((rows, n), 0.25, 1.0, seed=n)
+    _check_normalized(O.F32, n, x.astype(np.float64), (CudaArray.fromNumpy(x),))
+    x[0, n - 1], x[1, 0], x[2] = np.nan, np.inf, -np.inf
+    bad = CudaArray.fromNumpy(x)
+    for got in (bad.softmax(1).toNumpy(), bad.layerNorm([1], 1e-5).toNumpy()):
+        assert np.all(np.isnan(got[:3]).any(1)) and np.all(np.isfinite(got[3:]))
+
+
+def _check_normalized(dt, n, x, arrays):
+    from phptensors import CudaArray, synthetic
     u = 2.0 ** -53 if dt == O.F64 else 2.0 ** -24
     e = np.exp(x - x.max(1, keepdims=True))
     soft = e / e.sum(1, keepdims=True)
@@ -60,7 +96,7 @@ def test_ragged_softmax_and_layernorm(dt, n):
     pdt = "float64" if dt == O.F64 else "float32"
     ga, ba = CudaArray.fromNumpy(g.astype(pdt), pdt), CudaArray.fromNumpy(b.astype(pdt), pdt)
     norm = (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-5)
-    for a in (whole, view):
+    for a in arrays:
         # expf to 2 ulp, the sum's and the quotient's rounding
         got = a.softmax(1).toNumpy().astype(np.float64)
         assert np.allclose(got, soft, rtol=(16 + n ** 0.5) * u, atol=1e-30)
