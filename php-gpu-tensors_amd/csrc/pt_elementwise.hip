@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256) void k_where_vec(Opnd cond, Opnd x, Opnd y, vo
 }
 
 // Casts between the 32- and 16-bit floating types; V elements are 16 bytes
-// of the wider type.
+// of the narrower type.
 template <int DTI, int DTO>
 __global__ __launch_bounds__(256) void k_cast_vec(Opnd x, void *__restrict__ out, size_t total, unsigned cols)
 {
